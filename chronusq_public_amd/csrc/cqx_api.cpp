@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -20,6 +21,7 @@
 #include "cqx.h"
 #include "basis.hpp"
 #include "device_types.hpp"
+#include "eri_row.hpp"
 #include "kernels.hpp"
 #include "onebody.hpp"
 #include "ctx_access.hpp"
@@ -74,6 +76,11 @@ using cqx::PrimPair;
 using cqx::Quartet;
 
 namespace {
+
+// LDS of a row block beyond which a class pair takes quartet lists: all a
+// block can have (one block per CU still beats the lists: GHF (ps|ps) of
+// (H2O)16 1.41 against 2.04 ms)
+constexpr size_t kRowLdsUse = 160 * 1024;
 
 constexpr int kNumClass = (cqx::kMaxLDev + 1) * (cqx::kMaxLDev + 2) / 2;  // (la, lb), la >= lb
 inline int class_of(int la, int lb) { return la * (la + 1) / 2 + lb; }
@@ -156,6 +163,11 @@ struct cqx_ctx {
   std::vector<double> schwarz;                 // NS x NS
 
   DevBuf<PairRec> d_pairs[kNumClass];
+  // row kernels: ket records, columns of a row over the class's two angular
+  // momenta ([molecule][row_width], -1 padding)
+  DevBuf<cqx::RowKet> d_rowket[kNumClass];
+  DevBuf<int> d_colmap[kNumClass];
+  int row_width[kNumClass] = {};
   DevBuf<cqx::PairScr> d_scr[kNumClass];
   DevBuf<double> d_pn[kNumClass];  // per build: each pair's own block norms
   DevBuf<PrimPair> d_prims;
@@ -186,6 +198,8 @@ struct cqx_ctx {
   DevBuf<double> d_psum;
   DevBuf<double> d_store;
   DevBuf<long long> d_store_off;
+  DevBuf<double> d_jx, d_ja;                  // row kernels: Coulomb planes in pair order
+  DevBuf<double> d_rcount;                    // per row launch: quartets, candidates (integers), primitive sum
   DevBuf<long long> d_tidx, d_tot;  // candidate totals of an eager build, gathered for one copy
   // The workspace of the contraction group in flight: views of the buffers
   // above (allocated on demand) or of a fixed scratch region
@@ -203,7 +217,7 @@ struct cqx_ctx {
     cqx::ListLaunch *lists;
   } w{};
   size_t ws_scratch_peak = 0;  // bytes of the scratch region the last call used
-  hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_t0 = nullptr, ev_t1 = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_t0 = nullptr, ev_t1 = nullptr, ev_r0 = nullptr;
   // Concurrent class-pair launches (option "streams"): a build, eager or
   // recorded, deals its ERI launches round-robin over the context stream and
   // nstreams - 1 side streams, forked from and joined back into the context
@@ -230,6 +244,7 @@ struct cqx_ctx {
   std::vector<size_t> g_xoff, g_mnb2;  // per molecule: offset and size of its matrices
   std::vector<long long> g_cap;        // per class pair: candidate capacity
   std::vector<long long> g_lcap;       // per ERI slot: list capacity
+  std::vector<GraphSlot> g_rows;       // per row launch
   std::vector<GraphSlot> g_slots;      // per ERI slot (class pair, precision); la < 0: not launched
   DevBuf<cqx::ListLaunch> d_glists;
   DevBuf<long long> d_glstart, d_gidx, d_gchk;
@@ -241,6 +256,7 @@ struct cqx_ctx {
   // class, its member array (pair indices grouped by molecule and first
   // shell); per tile class pair, its sub-blocks, a range of d_sub.
   int use_tiles = 0;
+  int use_rows = 1;  // row kernels (option "rows")
   // lane-group classes that take tiles (bit k: k-th of ss|ss, ps|ss, ps|ps,
   // pp|ss, pp|ps, ds|ss, ds|ps, dp|ss); (ss|ss) and (dp|ss) are faster
   // through quartet lists
@@ -348,10 +364,8 @@ void make_prims(const cqx::Shell &A, const cqx::Shell &B, std::vector<PrimPair> 
       const double a = A.alpha[i], b = B.alpha[j], p = a + b;
       PrimPair pp;
       pp.p = p;
-      for (int d = 0; d < 3; ++d) {
-        pp.P[d] = (a * A.origin[d] + b * B.origin[d]) / p;
-        pp.PA[d] = pp.P[d] - A.origin[d];
-      }
+      pp.rp = 1.0 / p;
+      for (int d = 0; d < 3; ++d) pp.P[d] = (a * A.origin[d] + b * B.origin[d]) / p;
       pp.K = A.coef[i] * B.coef[j] * std::exp(-a * b / p * AB2);
       out.push_back(pp);
       if (alpha_a) alpha_a->push_back(a);
@@ -474,6 +488,7 @@ void setup_device_maps(cqx_ctx *c) {
 
 void upload_pairs(cqx_ctx *c);
 void build_tiles(cqx_ctx *c);
+void build_rows(cqx_ctx *c);
 
 // Significant pairs, primitive pairs and GPU Schwarz bounds.
 void build_pairs(cqx_ctx *c) {
@@ -602,8 +617,58 @@ void upload_pairs(cqx_ctx *c) {
     }
     c->d_scr[k].upload(scr, c->stream);
   }
+  build_rows(c);
   build_tiles(c);
   HIPCHK(hipStreamSynchronize(c->stream));
+}
+
+// Ket records and row columns of the row kernels.  A row over the kets
+// (c, d) of a class has one column per Cartesian function of c's angular
+// momentum in the molecule, and, when d's differs, one per function of that
+// (from the widest molecule's first part on).
+void build_rows(cqx_ctx *c) {
+  const cqx::Basis &B = c->basis;
+  std::vector<int> index(c->nbc);  // of a Cartesian function among those of its molecule and angular momentum
+  std::vector<std::array<std::vector<int>, cqx::kMaxLDev + 1>> funcs(c->nmol);
+  size_t most[cqx::kMaxLDev + 1] = {};
+  for (int m = 0; m < c->nmol; ++m) {
+    for (int s = B.mol_sh0[m]; s < B.mol_sh0[m + 1]; ++s)
+      for (int k = 0; k < cqx::ncart(B.shells[s].l); ++k) {
+        auto &f = funcs[m][B.shells[s].l];
+        index[B.bf_cart[s] + k] = (int)f.size();
+        f.push_back(B.bf_cart[s] + k - B.mol_bfc0[m]);
+      }
+    for (int l = 0; l <= cqx::kMaxLDev; ++l) most[l] = std::max(most[l], funcs[m][l].size());
+  }
+  for (int k = 0; k < kNumClass; ++k) {
+    if (c->cls[k].empty()) continue;
+    int lc, ld;
+    class_ls(k, lc, ld);
+    const int second = lc == ld ? 0 : (int)most[lc];
+    const int w = c->row_width[k] = (int)most[lc] + (lc == ld ? 0 : (int)most[ld]);
+    std::vector<int> map((size_t)c->nmol * w, -1);
+    for (int m = 0; m < c->nmol; ++m) {
+      std::copy(funcs[m][lc].begin(), funcs[m][lc].end(), map.begin() + (size_t)m * w);
+      if (lc != ld) std::copy(funcs[m][ld].begin(), funcs[m][ld].end(), map.begin() + (size_t)m * w + second);
+    }
+    std::vector<cqx::RowKet> v;
+    for (const PairRec &r : c->cls[k]) {
+      cqx::RowKet q{};
+      q.pp_off = r.pp_off;
+      q.npp = r.npp;
+      q.colc = (unsigned short)index[r.bfa + B.mol_bfc0[r.mol]];
+      q.cold = (unsigned short)(second + index[r.bfb + B.mol_bfc0[r.mol]]);
+      q.bfc = (unsigned short)r.bfa;
+      q.bfd = (unsigned short)r.bfb;
+      for (int d = 0; d < 3; ++d) {
+        q.C[d] = r.A[d];
+        q.CD[d] = r.AB[d];
+      }
+      v.push_back(q);
+    }
+    c->d_rowket[k].upload(v, c->stream);
+    c->d_colmap[k].upload(map, c->stream);
+  }
 }
 
 // Member arrays and sub-block tables of the tile path.  A class's pairs are
@@ -684,6 +749,27 @@ void build_tiles(cqx_ctx *c) {
   c->d_sub.upload(sub, c->stream);
 }
 
+// The counters of the row launches (quartets, candidates, primitive sum as a
+// double) into the call's statistics.
+void add_row_stats(cqx_ctx *c, const std::vector<cqx_ctx::GraphSlot> &slots,
+                   const std::vector<unsigned long long> &counts, bool pure_d, int w, int nJ, int nK) {
+  for (size_t k = 0; k < slots.size(); ++k) {
+    const auto &G = slots[k];
+    const unsigned long long *cnt = counts.data() + 3 * k;
+    double prim;
+    std::memcpy(&prim, cnt + 2, sizeof prim);
+    const double fl = class_pair_flops(G.la, G.lb, G.lc, G.ld, pure_d, prim, (double)cnt[0], w, nJ, nK);
+    c->stats.n_quartets += (long long)cnt[0];
+    c->stats.n_candidates += (long long)cnt[1];
+    c->stats.n_prim_quartets_max += (long long)prim;
+    c->stats.flops_model += fl;
+    if (G.f32) {
+      c->stats.n_quartets_f32 += (long long)cnt[0];
+      c->stats.flops_model_f32 += fl;
+    }
+  }
+}
+
 // Replay of the captured build for the densities of `list`: stage X and AX,
 // launch the graph, read back the candidate totals and list counts in one
 // synchronisation.  Returns false, with the caller's AX untouched, when a
@@ -707,11 +793,15 @@ bool replay_graph(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_comp
   HIPCHK(hipEventRecord(c->ev1, s));
   const size_t ncp = c->g_cap.size();
   std::vector<long long> tot(ncp);
-  std::vector<unsigned long long> counts(2 * ncp);
+  std::vector<unsigned long long> counts(2 * ncp), rcount(3 * c->g_rows.size());
   std::vector<double> psum(2 * ncp);
-  HIPCHK(hipMemcpyAsync(tot.data(), c->d_gchk.p, sizeof(long long) * ncp, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipMemcpyAsync(counts.data(), c->d_count.p, sizeof(unsigned long long) * 2 * ncp, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipMemcpyAsync(psum.data(), c->d_psum.p, sizeof(double) * 2 * ncp, hipMemcpyDeviceToHost, s));
+  if (ncp) {
+    HIPCHK(hipMemcpyAsync(tot.data(), c->d_gchk.p, sizeof(long long) * ncp, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(counts.data(), c->d_count.p, sizeof(unsigned long long) * 2 * ncp, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(psum.data(), c->d_psum.p, sizeof(double) * 2 * ncp, hipMemcpyDeviceToHost, s));
+  }
+  if (!rcount.empty())
+    HIPCHK(hipMemcpyAsync(rcount.data(), c->d_rcount.p, sizeof(double) * rcount.size(), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   for (size_t k = 0; k < ncp; ++k)
     if (tot[k] > c->g_cap[k]) return false;
@@ -742,6 +832,8 @@ bool replay_graph(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_comp
       c->stats.flops_model_f32 += fl;
     }
   }
+  c->stats.n_launch_eri += (int)c->g_rows.size();
+  add_row_stats(c, c->g_rows, rcount, c->g_pure_d, is_complex ? 2 : 1, c->g_nJ, c->g_nK);
   c->stats.graph = 2;
   return true;
 }
@@ -759,6 +851,7 @@ void init_ctx(cqx_ctx *c, const cqx::Basis &basis, double thresh, int device) {
   HIPCHK(hipEventCreate(&c->ev1));
   HIPCHK(hipEventCreate(&c->ev_t0));
   HIPCHK(hipEventCreate(&c->ev_t1));
+  HIPCHK(hipEventCreate(&c->ev_r0));
   HIPCHK(hipDeviceGetAttribute(&c->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
   c->ns = (int)c->basis.shells.size();
   c->nb = c->basis.nbasis;
@@ -968,6 +1061,7 @@ int cqx_ctx_destroy(cqx_ctx *c) {
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->ev_t0) (void)hipEventDestroy(c->ev_t0);
   if (c->ev_t1) (void)hipEventDestroy(c->ev_t1);
+  if (c->ev_r0) (void)hipEventDestroy(c->ev_r0);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   for (int i = 0; i < cqx_ctx::kMaxSide; ++i) {
     if (c->side[i]) (void)hipStreamSynchronize(c->side[i]);
@@ -1049,6 +1143,12 @@ int cqx_set_option(cqx_ctx *c, const char *name, double value) {
     // one Hermitian J and one Hermitian K plane; 0 (default): quartet lists
     if (!(value == 0.0 || value == 1.0 || value == 2.0)) return fail(c, CQX_ERR_ARG, "tiles must be 0, 1 or 2");
     c->use_tiles = (int)value;
+    return CQX_OK;
+  }
+  if (!std::strcmp(name, "rows")) {
+    // 1 (default): class pairs with a row kernel whose rows fit in LDS take
+    // it; 0: quartet lists for every class pair
+    c->use_rows = value != 0.0;
     return CQX_OK;
   }
   if (!std::strcmp(name, "tile_classes")) {
@@ -1240,6 +1340,7 @@ size_t workspace_bytes(const cqx_ctx *c) {
   add(c->d_lstart); add(c->d_molmax); add(c->d_molplanes); add(c->d_quart); add(c->d_count);
   add(c->d_psum); add(c->d_tidx); add(c->d_tot); add(c->d_acc_tune); add(c->d_molplanes_tune);
   add(c->d_glists); add(c->d_glstart); add(c->d_gidx); add(c->d_gchk);
+  add(c->d_jx); add(c->d_ja); add(c->d_rcount);
   add(c->d_tiles); add(c->d_tcount); add(c->d_tpsum); add(c->d_tll); add(c->d_tstart);
   for (int k = 0; k < kNumClass; ++k) add(c->d_pn[k]);
   return b;
@@ -1463,12 +1564,54 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           if (tc->cb == cb && tc->ck == ck) return true;
         return false;
       };
+      // row class pairs: the row planes of every exchange contraction and
+      // the Coulomb planes, when they and the rows fit a block's LDS
+      struct RowCP { int cb, ck; };
+      std::vector<RowCP> rcps;
+      cqx::RowLaunch row0{};
+      for (int p = 0; p < (int)pd.size(); ++p) {
+        const int k = pd[p].kind;
+        if (k == cqx::kJHer || k == cqx::kJNonHer) {
+          if (row0.nj < cqx::kRowJ) {
+            row0.jmat[row0.nj] = pd[p].m;
+            row0.jcoef[row0.nj] = k == cqx::kJHer ? 1.0 : 0.5;
+          }
+          ++row0.nj;
+        } else {
+          // a Hermitian plane by columns (conjugated), a non-Hermitian one both ways
+          for (int colwise = 1; colwise >= (k == cqx::kKHer ? 1 : 0); --colwise) {
+            if (row0.nk < cqx::kRowPlanes) row0.k[row0.nk] = {k, pidx[p], colwise, pd[p].m, pd[p].sign};
+            ++row0.nk;
+          }
+        }
+      }
+      const bool rows_ok = c->use_rows && !scr && !c->fast_lanes && row0.nj <= cqx::kRowJ &&
+                           row0.nk <= cqx::kRowPlanes && *std::max_element(mnbc.begin(), mnbc.end()) <= 0xFFFF;
+      auto row_fits = [&](int cb, int ck) {
+        int la_, lb_, lc_, ld_;
+        class_ls(cb, la_, lb_);
+        class_ls(ck, lc_, ld_);
+        const int ncq = cqx::ncart(la_) * cqx::ncart(lb_) * cqx::ncart(lc_) * cqx::ncart(ld_);
+        if (!(ncq <= c->fast_max_nc || (c->use_wave && c->fast_max_nc > 0))) return false;
+        const size_t b = cqx::eri_row_lds(la_, lb_, lc_, ld_, 0, row0.nk, c->row_width[ck]);
+        return b > 0 && b <= (size_t)kRowLdsUse;
+      };
+      if (rows_ok)
+        for (int cb = 0; cb < kNumClass; ++cb)
+          for (int ck = 0; ck <= cb; ++ck)
+            if (!c->cls[cb].empty() && !c->cls[ck].empty() && !is_tile_cp(cb, ck) && row_fits(cb, ck))
+              rcps.push_back({cb, ck});
+      auto is_row_cp = [&](int cb, int ck) {
+        for (const auto &rc : rcps)
+          if (rc.cb == cb && rc.ck == ck) return true;
+        return false;
+      };
       struct CP { int cb, ck, nbra; long long ncand; size_t coff; std::vector<long long> off; };
       std::vector<CP> cps;
       size_t cand_total = 0;
       for (int cb = 0; cb < kNumClass; ++cb)
         for (int ck = 0; ck <= cb; ++ck) {
-          if (c->cls[cb].empty() || c->cls[ck].empty() || is_tile_cp(cb, ck)) continue;
+          if (c->cls[cb].empty() || c->cls[ck].empty() || is_tile_cp(cb, ck) || is_row_cp(cb, ck)) continue;
           CP cp{cb, ck, (int)c->cls[cb].size(), 0, cand_total, {}};
           cand_total += (size_t)cp.nbra + 1;
           cps.push_back(std::move(cp));
@@ -1538,6 +1681,146 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       front();
       const bool mixed = c->fp32_cut > 0.0;
       const int qmul = mixed ? 2 : 1;  // quartet lists per class pair
+      // side streams for concurrent class-pair launches: created outside any
+      // capture, forked from the context stream before the launches and
+      // joined back into it after them (also inside a recorded build); the
+      // allocation-free path launches on the context stream alone
+      auto ensure_side = [&](int nst) {
+        for (int i = 0; i < nst - 1; ++i)
+          if (!c->side[i]) {
+            HIPCHK(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
+            HIPCHK(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
+          }
+        if (nst > 1 && !c->ev_fork) HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+      };
+      auto fork_side = [&](int nst) {
+        if (nst <= 1) return;
+        HIPCHK(hipEventRecord(c->ev_fork, s));
+        for (int i = 0; i < nst - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
+      };
+      auto join_side = [&](int nst) {
+        for (int i = 0; i < nst - 1; ++i) {
+          HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
+          HIPCHK(hipStreamWaitEvent(s, c->ev_join[i], 0));
+        }
+      };
+      auto stream_of = [&](int launch, int nst) { return launch % nst == 0 ? s : c->side[launch % nst - 1]; };
+      const bool tuning = c->autotune_pending && !scr;  // the allocation-free path never times
+      const int nst_all = (tuning || scr) ? 1 : c->nstreams;
+      // --- row class pairs: Coulomb planes to pair order, then every launch;
+      // beside quartet lists they go to the side streams only, so that the
+      // list building on the context stream need not wait for them ---
+      const int nrow = (int)rcps.size();
+      size_t joff[kNumClass + 1] = {};
+      std::vector<cqx_ctx::GraphSlot> row_slots;
+      std::vector<unsigned long long> rcount;  // per launch: quartets, candidates, primitive sum (a double)
+      auto pair_order = [&](int k) {
+        cqx::PairOrder po{};
+        int la_, lb_;
+        class_ls(k, la_, lb_);
+        po.pairs = c->d_pairs[k].p;
+        po.npair = (int)c->cls[k].size();
+        po.na = cqx::ncart(la_);
+        po.nb = cqx::ncart(lb_);
+        po.m0 = mp[0];
+        po.mols = w.molplanes;
+        po.nmol = nmol;
+        for (int p = 0; p < (int)pd.size(); ++p)
+          if (pd[p].kind == cqx::kJHer || pd[p].kind == cqx::kJNonHer) {
+            po.kind[po.nj] = pd[p].kind;
+            po.idx[po.nj] = pidx[p];
+            po.stride[po.nj++] = ps.kps[pd[p].kind];
+          }
+        po.jx = c->d_jx.p + joff[k];
+        po.ja = c->d_ja.p + joff[k];
+        return po;
+      };
+      if (nrow) {
+        for (int k = 0; k < kNumClass; ++k) {
+          int la_, lb_;
+          class_ls(k, la_, lb_);
+          joff[k + 1] = joff[k] + (size_t)row0.nj * cqx::ncart(la_) * cqx::ncart(lb_) * c->cls[k].size();
+        }
+        const size_t nslot = (size_t)nrow * qmul;
+        c->d_jx.ensure(std::max<size_t>(joff[kNumClass], 1));
+        c->d_ja.ensure(std::max<size_t>(joff[kNumClass], 1));
+        c->d_rcount.ensure(3 * nslot);
+        rcount.resize(3 * nslot);
+        ensure_side(nst_all);
+      }
+      auto rows_front = [&]() {
+        if (!nrow) return;
+        HIPCHK(cqx::launch_zero(c->d_rcount.p, rcount.size(), s));
+        HIPCHK(cqx::launch_zero(c->d_ja.p, joff[kNumClass], s));
+        for (int k = 0; k < kNumClass; ++k)
+          if (!c->cls[k].empty() && row0.nj) HIPCHK(cqx::launch_pair_pack(pair_order(k), s));
+      };
+      // every row launch; stream(k): the stream of the k-th
+      auto rows_launch = [&](const std::function<hipStream_t(int)> &stream) {
+        int nl = 0;
+        for (int f = 0; f < qmul; ++f)
+          for (int r = 0; r < nrow; ++r) {
+            const int cb = rcps[r].cb, ck = rcps[r].ck;
+            cqx::RowLaunch R = row0;
+            class_ls(cb, R.la, R.lb);
+            class_ls(ck, R.lc, R.ld);
+            R.bra = c->d_pairs[cb].p;
+            R.bscr = c->d_scr[cb].p;
+            R.kscr = c->d_scr[ck].p;
+            R.ket = c->d_rowket[ck].p;
+            R.nbra = (int)c->cls[cb].size();
+            R.nket = (int)c->cls[ck].size();
+            int longest = 0;
+            for (int m = 0; m < nmol; ++m) longest = std::max(longest, c->seg[ck][m + 1] - c->seg[ck][m]);
+            R.nchunk = (longest + cqx::kRowChunk - 1) / cqx::kRowChunk;
+            R.seg = c->d_seg.p + (size_t)ck * (nmol + 1);
+            R.same_class = cb == ck;
+            R.bra_pn = w.pn[cb];
+            R.ket_pn = w.pn[ck];
+            R.Bg = w.Bg;
+            R.Bm = w.Bm;
+            R.molmax = w.molmax;
+            R.mol_boff = c->d_mol_boff.p;
+            R.mol_ns = c->d_mol_ns.p;
+            R.nmat = nmat;
+            R.thresh = c->thresh;
+            R.screen = screen;
+            R.cut32 = mixed ? c->fp32_cut : 0.0;
+            R.fp32 = f;
+            R.prims = c->d_prims.p;
+            R.primc32 = c->d_primc32.p;
+            R.rys = c->d_rys.p;
+            R.rys32 = c->d_rys32.p;
+            R.m0 = mp[0];
+            R.mols = w.molplanes;
+            R.nmol = nmol;
+            for (int k = 0; k < 4; ++k) R.kps[k] = ps.kps[k];
+            R.width = c->row_width[ck];
+            R.colmap = c->d_colmap[ck].p;
+            R.jx_bra = c->d_jx.p + joff[cb];
+            R.jx_ket = c->d_jx.p + joff[ck];
+            R.ja_bra = c->d_ja.p + joff[cb];
+            R.ja_ket = c->d_ja.p + joff[ck];
+            double *cnt = c->d_rcount.p + 3 * ((size_t)f * nrow + r);
+            R.count = reinterpret_cast<unsigned long long *>(cnt);
+            R.prim_sum = cnt + 2;
+            HIPCHK(cqx::launch_eri_row(R, stream(nl++)));
+          }
+        return nl;
+      };
+      auto rows_back = [&]() {
+        if (nrow && row0.nj)
+          for (int k = 0; k < kNumClass; ++k)
+            if (!c->cls[k].empty()) HIPCHK(cqx::launch_pair_unpack(pair_order(k), s));
+      };
+      rows_front();
+      if (nrow) {
+        HIPCHK(hipEventRecord(c->ev_r0, s));
+        fork_side(nst_all);
+        c->stats.n_launch_eri += rows_launch([&](int k) {
+          return nst_all == 1 ? s : cps.empty() ? stream_of(k, nst_all) : c->side[k % (nst_all - 1)];
+        });
+      }
       // tile lists of the tile class pairs: one launch over their sub-blocks;
       // each sub-block gives at most one tile per precision
       const int nt = (int)tcps.size();
@@ -1594,7 +1877,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         HIPCHK(cqx::launch_gather(w.cand, w.tidx, (int)cps.size(), w.tot, s));
         HIPCHK(hipMemcpyAsync(totals.data(), w.tot, sizeof(long long) * cps.size(), hipMemcpyDeviceToHost, s));
       }
-      HIPCHK(hipStreamSynchronize(s));
+      if (nt || !cps.empty()) HIPCHK(hipStreamSynchronize(s));
       // entries of one list batch: the option, or what the scratch region
       // leaves after this group's fixed workspace (less a reserve for the
       // per-batch tables)
@@ -1703,30 +1986,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       auto launch_eri = [&](const cqx::EriLaunch &E, hipStream_t st) {
         launch_family(E, route(E.la, E.lb, E.lc, E.ld, E.fp32), st);
       };
-      // side streams for concurrent class-pair launches: created outside any
-      // capture, forked from the context stream before the launches and
-      // joined back into it after them (also inside a recorded build); the
-      // allocation-free path launches on the context stream alone
-      auto ensure_side = [&](int nst) {
-        for (int i = 0; i < nst - 1; ++i)
-          if (!c->side[i]) {
-            HIPCHK(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
-            HIPCHK(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
-          }
-        if (nst > 1 && !c->ev_fork) HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-      };
-      auto fork_side = [&](int nst) {
-        if (nst <= 1) return;
-        HIPCHK(hipEventRecord(c->ev_fork, s));
-        for (int i = 0; i < nst - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
-      };
-      auto join_side = [&](int nst) {
-        for (int i = 0; i < nst - 1; ++i) {
-          HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
-          HIPCHK(hipStreamWaitEvent(s, c->ev_join[i], 0));
-        }
-      };
-      auto stream_of = [&](int launch, int nst) { return launch % nst == 0 ? s : c->side[launch % nst - 1]; };
       // --- back to pure functions, symmetrise, accumulate into AX: the
       // contractions' transforms are independent and are dealt over nst
       // streams like the ERI launches (side streams already created) ---
@@ -1789,7 +2048,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       // build (they size the launches of a recorded graph)
       std::vector<double> cp_count(2 * cps.size(), 0.0), cp_psum(2 * cps.size(), 0.0);
       bool tune_ready = false;
-      const bool tuning = c->autotune_pending && !scr;  // the allocation-free path never times
       cqx::PlaneSet ps_tune = ps;
       // scratch accumulators for the timing launches of the autotuner
       auto prepare_tune = [&]() {
@@ -1837,7 +2095,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       // ERI + digestion of the tile lists: launched with the first batch's
       // ERI launches (or alone when no quartet list remains), each over its
       // list's capacity (empty tiles exit at once)
-      const int nst_all = (tuning || scr) ? 1 : c->nstreams;
       bool tiles_done = nt == 0;
       auto launch_tiles = [&](int nst, int &nl) {
         tiles_done = true;
@@ -2038,6 +2295,12 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         eri_ms_total += ms;
       }
       ensure_side(nst_all);
+      if (nrow) {
+        join_side(nst_all);
+        HIPCHK(hipEventRecord(c->ev1, s));
+        HIPCHK(hipMemcpyAsync(rcount.data(), c->d_rcount.p, sizeof(double) * rcount.size(), hipMemcpyDeviceToHost, s));
+        rows_back();
+      }
       back(nst_all);
       if (!scr) {
         const hipMemcpyKind dk = mem == CQX_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
@@ -2047,6 +2310,21 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
                                   sizeof(double) * mnb2[m] * ew, dk, s));
       }
       HIPCHK(hipStreamSynchronize(s));
+      if (nrow) {
+        float ms = 0.0f;  // with the list launches beside the row launches
+        HIPCHK(hipEventElapsedTime(&ms, c->ev_r0, c->ev1));
+        eri_ms_total = ms;
+        row_slots.clear();
+        for (int f = 0; f < qmul; ++f)
+          for (const auto &rc : rcps) {
+            cqx_ctx::GraphSlot G{};
+            class_ls(rc.cb, G.la, G.lb);
+            class_ls(rc.ck, G.lc, G.ld);
+            G.f32 = f;
+            row_slots.push_back(G);
+          }
+        add_row_stats(c, row_slots, rcount, pure_d, is_complex ? 2 : 1, nJ, nK);
+      }
       if (scr) scratch_peak = std::max(scratch_peak, scr->used);
       // Record the same build into a graph for the next calls (option
       // graph; one contraction group and one list batch).  Capacities are
@@ -2069,7 +2347,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           lcap[ncp + k] = (long long)std::ceil(cp_count[ncp + k] * c->graph_margin) + 1024;
       }
       for (size_t kk = 0; kk < 2 * ncp; ++kk) lseg[kk + 1] = lseg[kk] + lcap[kk];
-      if (!scr && c->use_graph && start == 0 && nmat == nper && batches.size() == 1 && ncp > 0 &&
+      if (!scr && c->use_graph && start == 0 && nmat == nper && batches.size() == 1 && (ncp > 0 || nrow > 0) &&
           lseg[2 * ncp] <= c->list_cap * qmul) {
         c->d_quart.ensure((size_t)lseg[2 * ncp]);
         c->d_count.ensure(2 * ncp);
@@ -2123,7 +2401,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         c->d_glists.upload(gl, s);
         c->d_glstart.upload(glst, s);
         c->d_gidx.upload(gidx, s);
-        c->d_gchk.ensure(ncp);
+        c->d_gchk.ensure(std::max<size_t>(ncp, 1));
         const int nst = c->nstreams;
         ensure_side(nst);
         HIPCHK(hipStreamSynchronize(s));  // every upload done before recording
@@ -2132,12 +2410,13 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         bool forked = false;
         try {
           front();
+          rows_front();
           HIPCHK(cqx::launch_zero(reinterpret_cast<double *>(w.count), 2 * ncp, s));
           HIPCHK(cqx::launch_zero(w.psum, 2 * ncp, s));
           HIPCHK(cqx::launch_quartet_lists(c->d_glists.p, c->d_glstart.p, (int)ncp, glst[ncp], s));
           fork_side(nst);
           forked = true;
-          int nlaunched = 0;
+          int nlaunched = nrow ? rows_launch([&](int k) { return stream_of(k, nst); }) : 0;
           for (size_t kk = 0; kk < 2 * ncp; ++kk) {
             if (slots[kk].la < 0) continue;
             const size_t k = kk % ncp;
@@ -2153,6 +2432,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           }
           join_side(nst);
           forked = false;
+          rows_back();
           back(nst);
           HIPCHK(cqx::launch_gather(w.cand, c->d_gidx.p, (int)ncp, c->d_gchk.p, s));
         } catch (...) {
@@ -2184,6 +2464,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         c->g_cap = gcap;
         c->g_lcap = lcap;
         c->g_slots = slots;
+        c->g_rows = row_slots;
         c->stats.graph = 1;
       }
       start += nmat;
@@ -2305,6 +2586,15 @@ int cqx_scratch_size(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_c
     b += 2 * planes * sizeof(double);                // Cartesian planes and accumulators
     if (c->autotune_pending) b += planes * sizeof(double) + nmol * sizeof(cqx::MolPlanes);
     b += 2 * nmol * sizeof(cqx::MolPlanes);
+    if (c->use_rows) {  // Coulomb planes in pair order and counters of the row kernels
+      size_t pc = 0;
+      for (int k = 0; k < kNumClass; ++k) {
+        int la, lb;
+        class_ls(k, la, lb);
+        pc += (size_t)cqx::ncart(la) * cqx::ncart(lb) * c->cls[k].size();
+      }
+      b += 2 * sizeof(double) * std::max<size_t>(cqx::kRowJ * pc, 1) + 3 * qmul * (ncp + 1) * sizeof(double);
+    }
     b += cand * (sizeof(long long) + sizeof(int)) + scan;
     b += 2 * ncp * sizeof(long long);                // gathered candidate totals
     b += (size_t)quart * sizeof(Quartet);            // quartet lists

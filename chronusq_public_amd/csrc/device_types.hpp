@@ -24,6 +24,18 @@ struct PairRec {
   double A[3];     // centre of shell a
 };
 
+// What the row kernels read of a ket pair (64 bytes): its primitive pairs,
+// its first functions and their columns in the bra's rows (see RowLaunch),
+// the centre C and C - D.  For one class on both shells the columns
+// are equal exactly when c and d are the same shell.
+struct alignas(16) RowKet {
+  int pp_off, npp;
+  unsigned short colc, cold;  // columns
+  unsigned short bfc, bfd;    // first Cartesian functions within the molecule
+  double C[3];
+  double CD[3];
+};
+
 // What the quartet screen reads of a shell pair, 16 bytes: shells s1, s2
 // (numbered within the molecule) in the low and high 16 bits of s12, the
 // contraction-length product Ka Kb, the molecule and the Schwarz bound.
@@ -34,12 +46,13 @@ struct PairScr {
   double Q;
 };
 
-// One surviving primitive pair of a shell pair (kernel orientation).
-struct PrimPair {
+// One surviving primitive pair of a shell pair (kernel orientation): three
+// 16-byte loads.  P - A is formed from the shell pair's A.
+struct alignas(16) PrimPair {
   double p;        // alpha_a + alpha_b
-  double P[3];     // Gaussian product centre
-  double PA[3];    // P - A
   double K;        // c_a c_b exp(-alpha_a alpha_b / p |AB|^2)
+  double P[3];     // Gaussian product centre
+  double rp;       // 1 / p
 };
 
 // A primitive pair as the FP32 lists read it, in one 16-byte load: with b

@@ -1,0 +1,473 @@
+// Row kernels: screening, ERI evaluation and J/K digestion of one class pair
+// in one launch, for the classes whose contracted Cartesian quartet fits a
+// lane's registers.
+//
+// What bounded the quartet-list kernels: their J/K updates went to HBM as
+// memory-side atomics (7 to 15 per quartet, executed at about 24 per ns on
+// this device whatever the kernel does), and the updates were formed by the
+// whole wave from quartets staged in LDS, with as much index arithmetic and
+// LDS latency per update as arithmetic.  Here a block takes one bra pair
+// (a, b) and a chunk of its kets.  For a fixed bra every exchange update
+// falls into the rows K(a, :) and K(b, :), and every density element read
+// comes from the rows X(a, :) and X(b, :): both sit in LDS for the whole
+// chunk, in columns numbered over the functions of the ket class's two
+// angular momenta only.  A lane (or a group of G lanes that split the ket's
+// primitive pairs) evaluates a ket and digests it from its registers with
+// LDS atomics; the rows go to HBM once per chunk.  J(a, b) is summed over
+// the wave; J(c, d) and X(d, c) are kept in the class's pair order, in which
+// neighbouring lanes hold neighbouring doubles.
+//
+// Each block screens its own kets (no quartet list, no host round trip) and
+// sorts the survivors into two bins by contraction length, the long ones
+// with more lanes per ket, so that a wave's lanes have similar loops.
+//
+// Measured against the quartet-list build (ms a build): C40H82 / 6-31G(d)
+// FP64 90.5 -> 36.9, mixed 71.5 -> 30.8; 32 water clusters batched, mixed,
+// 75 -> 38; GHF (H2O)16 / cc-pVDZ 12.8 -> 9.4; non-Hermitian complex (H2O)7
+// 3.2 -> 2.0; (H2O)4 1.38 -> 1.10.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "digest.hpp"
+#include <mutex>
+
+#include "digest.hpp"
+#include "eri_bra.hpp"
+#include "eri_class.hpp"
+#include "eri_row.hpp"
+#include "screen.hpp"
+
+namespace cqx {
+
+namespace {
+
+// contraction-length product above which a ket goes to the long bin
+constexpr int kRowLongKet = 8;
+
+// sum over the wave, in every lane
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+
+__device__ __forceinline__ int pow2_at_least(int n) {
+  int p = 1;
+  while (p < n) p *= 2;
+  return p;
+}
+
+// The four exchange updates of one quartet in row form: with rows Xa = X(a, :)
+// and Xb = X(b, :),
+//   K(a, c) += I X(b, d)   K(a, d) += I X(b, c)
+//   K(b, c) += I X(a, d)   K(b, d) += I X(a, c)
+// (direct.hpp:1889-1917, 1961-1998; the 1/2 is applied when the rows are
+// flushed).  k: the plane's NA + NB exchange rows of w columns, kets at
+// columns c and d; x(r, k, second): element k of row r from ket shell c or d.
+template <class K, class X>
+__device__ __forceinline__ void digest_rows(const double (&I)[K::NC], const X &x, double *k, int w, int c, int d) {
+  {
+    double kc[K::NCA][K::NCC], kd[K::NCA][K::NCD];
+#pragma unroll
+    for (int ia = 0; ia < K::NCA; ++ia) {
+#pragma unroll
+      for (int ic = 0; ic < K::NCC; ++ic) kc[ia][ic] = 0.0;
+#pragma unroll
+      for (int id = 0; id < K::NCD; ++id) kd[ia][id] = 0.0;
+    }
+#pragma unroll
+    for (int ib = 0; ib < K::NCB; ++ib) {
+      double xc[K::NCC], xd[K::NCD];
+#pragma unroll
+      for (int ic = 0; ic < K::NCC; ++ic) xc[ic] = x(K::NCA + ib, ic, false);
+#pragma unroll
+      for (int id = 0; id < K::NCD; ++id) xd[id] = x(K::NCA + ib, id, true);
+#pragma unroll
+      for (int ia = 0; ia < K::NCA; ++ia)
+#pragma unroll
+        for (int ic = 0; ic < K::NCC; ++ic)
+#pragma unroll
+          for (int id = 0; id < K::NCD; ++id) {
+            const double v = I[K::oidx(ia, ib, ic, id)];
+            kc[ia][ic] = fma(v, xd[id], kc[ia][ic]);
+            kd[ia][id] = fma(v, xc[ic], kd[ia][id]);
+          }
+    }
+#pragma unroll
+    for (int ia = 0; ia < K::NCA; ++ia) {
+#pragma unroll
+      for (int ic = 0; ic < K::NCC; ++ic) unsafeAtomicAdd(k + ia * w + c + ic, kc[ia][ic]);
+#pragma unroll
+      for (int id = 0; id < K::NCD; ++id) unsafeAtomicAdd(k + ia * w + d + id, kd[ia][id]);
+    }
+  }
+#pragma unroll
+  for (int ib = 0; ib < K::NCB; ++ib) {
+    double kc[K::NCC], kd[K::NCD];
+#pragma unroll
+    for (int ic = 0; ic < K::NCC; ++ic) kc[ic] = 0.0;
+#pragma unroll
+    for (int id = 0; id < K::NCD; ++id) kd[id] = 0.0;
+#pragma unroll
+    for (int ia = 0; ia < K::NCA; ++ia) {
+      double xc[K::NCC], xd[K::NCD];
+#pragma unroll
+      for (int ic = 0; ic < K::NCC; ++ic) xc[ic] = x(ia, ic, false);
+#pragma unroll
+      for (int id = 0; id < K::NCD; ++id) xd[id] = x(ia, id, true);
+#pragma unroll
+      for (int ic = 0; ic < K::NCC; ++ic)
+#pragma unroll
+        for (int id = 0; id < K::NCD; ++id) {
+          const double v = I[K::oidx(ia, ib, ic, id)];
+          kc[ic] = fma(v, xd[id], kc[ic]);
+          kd[id] = fma(v, xc[ic], kd[id]);
+        }
+    }
+    double *row = k + (K::NCA + ib) * w;
+#pragma unroll
+    for (int ic = 0; ic < K::NCC; ++ic) unsafeAtomicAdd(row + c + ic, kc[ic]);
+#pragma unroll
+    for (int id = 0; id < K::NCD; ++id) unsafeAtomicAdd(row + d + id, kd[id]);
+  }
+}
+
+// Work item t of a launch: bra pair t / nchunk, candidate kets
+// [t % nchunk, ...) kRowChunk of its molecule's segment.  Dynamic LDS: the
+// exchange rows ([plane][NA + NB][width]), then, with XL, the density rows;
+// without XL the density is read from its planes in global memory (many
+// planes, whose density rows would not fit beside the exchange rows).
+template <class K>
+constexpr int row_threads() {
+  return K::NC > 54 ? 256 : 512;
+}
+template <int LA, int LB, int LC, int LD, class R, bool XL>
+__global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_kernel(RowLaunch a) {
+  using K = Cls<LA, LB, LC, LD>;
+  constexpr int kRowThreads = row_threads<K>();
+  constexpr int NROW = K::NCA + K::NCB, NAB = K::NCA * K::NCB, NCD = K::NCC * K::NCD;
+  extern __shared__ double s_rows[];
+  __shared__ R s_tab[rys_tab_len(K::NR)];
+  __shared__ unsigned s_queue[kRowChunk];  // short kets from the front, long ones from the back
+  __shared__ double s_jab[kRowJ * NAB];
+  __shared__ int s_n[2], s_next;
+  __shared__ unsigned long long s_tot[2];
+  __shared__ double s_psum;
+  const int tid = threadIdx.x, lane = tid & 63;
+  {
+    const R *g = rys_table<R>(a.rys, a.rys32) + rys_tab_off(K::NR);
+    for (int e = tid; e < rys_tab_len(K::NR); e += kRowThreads) s_tab[e] = g[e];
+    if (tid == 0) {
+      s_tot[0] = s_tot[1] = 0;
+      s_psum = 0.0;
+    }
+  }
+  const int w = a.width, rows = a.nk * NROW * w;
+  double *s_k = s_rows, *s_x = s_rows + rows;
+  const long long nitem = (long long)a.nbra * a.nchunk;
+  for (long long item = blockIdx.x; item < nitem; item += gridDim.x) {
+    const int i = (int)(item / a.nchunk), ch = (int)(item - (long long)i * a.nchunk);
+    const ConstPtr<PairRec> bp = as_const(a.bra + i);
+    const int mol = bp->mol;
+    const int lo = as_const(a.seg)[mol];
+    int hi = as_const(a.seg)[mol + 1];
+    if (a.same_class) hi = min(hi, i + 1);
+    const int j0 = lo + ch * kRowChunk, j1 = min(hi, j0 + kRowChunk);
+    if (j0 >= j1) continue;
+    // candidates: the Schwarz pre-cut prefix of the molecule's kets (Q
+    // descending), as in cand_count_kernel; the precision split is monotonic
+    // in the ket index too
+    const double Qi = bp->Q;
+    double need = 0.0;
+    if (a.screen) {
+      const double bmax = as_const(a.molmax)[mol];
+      if (bmax * Qi * as_const(a.kscr + lo)->Q < a.thresh) continue;
+      need = a.thresh / (bmax * Qi);
+      if (as_const(a.kscr + j0)->Q < need) continue;
+    }
+    if (a.cut32 > 0.0) {
+      if (!a.fp32 && Qi * as_const(a.kscr + j0)->Q < a.cut32) continue;
+      if (a.fp32 && !(Qi * as_const(a.kscr + (j1 - 1))->Q < a.cut32)) continue;
+    }
+    __syncthreads();  // the previous item's rows, queue and sums have been read
+    if (tid == 0) {
+      s_n[0] = s_n[1] = 0;
+      s_next = 0;
+    }
+    __syncthreads();
+    const PairScr P = a.bscr[i];
+    const ScreenArgs sa{a.Bg, a.Bm, a.mol_boff, a.mol_ns, a.nmat, a.thresh, a.screen};
+    int ncand = 0;
+    double psum = 0.0;
+    for (int t = tid; t < kRowChunk; t += kRowThreads) {
+      const int j = j0 + t;
+      bool pass = false, cand = false;
+      unsigned mask = 0;
+      int kk = 0;
+      if (j < j1) {
+        const PairScr Q = a.kscr[j];
+        const double qq = P.Q * Q.Q;
+        kk = Q.kk;
+        const bool lo32 = a.cut32 > 0.0 && qq < a.cut32;
+        if (lo32 == (a.fp32 != 0) && (!a.screen || Q.Q >= need)) {
+          cand = true;
+          pass = screen_candidate(sa, P, Q, a.bra_pn + (size_t)i * (a.nmat + 1), a.ket_pn + (size_t)j * (a.nmat + 1),
+                                  qq, mask);
+        }
+      }
+      ncand += __popcll(__ballot(cand));
+      if (pass) psum += (double)P.kk * (double)kk;
+      const bool lng = kk > kRowLongKet;
+      const unsigned long long b0 = __ballot(pass && !lng), b1 = __ballot(pass && lng);
+      int p0 = 0, p1 = 0;
+      if (lane == 0) {
+        if (b0) p0 = atomicAdd(&s_n[0], (int)__popcll(b0));
+        if (b1) p1 = atomicAdd(&s_n[1], (int)__popcll(b1));
+      }
+      p0 = __shfl(p0, 0);
+      p1 = __shfl(p1, 0);
+      const unsigned long long below = (1ull << lane) - 1ull;
+      if (pass && !lng) s_queue[p0 + __popcll(b0 & below)] = (unsigned)t | (mask << 16);
+      if (pass && lng) s_queue[kRowChunk - 1 - (p1 + __popcll(b1 & below))] = (unsigned)t | (mask << 16);
+    }
+    psum = wave_sum(psum);
+    if (lane == 0) {
+      if (ncand) atomicAdd(&s_tot[1], (unsigned long long)ncand);
+      if (psum != 0.0) unsafeAtomicAdd(&s_psum, psum);
+    }
+    __syncthreads();
+    const int n0 = s_n[0], n1 = s_n[1];
+    if (n0 + n1 == 0) continue;
+    if (tid == 0) s_tot[0] += (unsigned long long)(n0 + n1);
+    // the molecule's planes; density rows in, exchange rows cleared
+    const bool one = a.nmol == 1;
+    const ConstPtr<MolPlanes> mp = as_const(a.mols + (one ? 0 : mol));
+    const int N = one ? a.m0.nbc : mp->nbc;
+    const int bfa = bp->bfa, bfb = bp->bfb;
+    const int *colmap = a.colmap + (size_t)mol * w;
+    for (int p = 0; p < a.nk; ++p) {
+      const RowPlane &rp = a.k[p];
+      const GlobalDouble *x = (const GlobalDouble *)(one ? a.m0.kx[rp.kind] : mp->kx[rp.kind]) + rp.idx;
+      const int S = a.kps[rp.kind];
+      double *xs = s_x + p * NROW * w, *ks = s_k + p * NROW * w;
+      for (int c = tid; c < w; c += kRowThreads) {
+        const int f = colmap[c];
+        if (f < 0) continue;
+#pragma unroll
+        for (int r = 0; r < NROW; ++r) {
+          const int fr = r < K::NCA ? bfa + r : bfb + (r - K::NCA);
+          if constexpr (XL)
+            xs[r * w + c] = rp.sign * x[(size_t)(rp.colwise ? f + (size_t)fr * N : fr + (size_t)f * N) * S];
+          ks[r * w + c] = 0.0;
+        }
+      }
+    }
+    for (int e = tid; e < a.nj * NAB; e += kRowThreads) s_jab[e] = 0.0;
+    __syncthreads();
+    // lanes per ket of each bin: enough for the block's lanes when there are
+    // few kets, and for at most about 128 primitive quartets per lane
+    const int nb = bp->npp;
+    int g0 = 1, g1 = 4;
+    while (g0 < 8 && (n0 * g0 < kRowThreads || nb * (kRowLongKet / g0) > 128)) g0 *= 2;
+    while (g1 < 16 && (n1 * g1 < kRowThreads || nb * (32 / g1) > 128)) g1 *= 2;
+    const int ng1 = (n1 * g1 + 63) >> 6, ng0 = (n0 * g0 + 63) >> 6;
+    const int pa = bp->a, pb = bp->b;
+    const double bra_scale = 0.5 * (pa == pb ? 1.0 : 2.0);
+    for (;;) {
+      int grp = 0;
+      if (lane == 0) grp = atomicAdd(&s_next, 1);
+      grp = __builtin_amdgcn_readfirstlane(grp);
+      if (grp >= ng0 + ng1) break;
+      const bool lng = grp < ng1;
+      const int G = lng ? g1 : g0, nbin = lng ? n1 : n0;
+      const int lg = __builtin_ctz(G);
+      const int slot = ((lng ? grp : grp - ng1) << (6 - lg)) + (lane >> lg), g = lane & (G - 1);
+      const bool valid = slot < nbin;
+      const unsigned q = valid ? s_queue[lng ? kRowChunk - 1 - slot : slot] : 0u;
+      const int j = j0 + (int)(q & 0xFFFFu);
+      const unsigned mask = q >> 16;
+      int koff = 0, nkp = 0, c = 0, d = 0, fc = 0, fd = 0;
+      double Cc[3] = {}, CD[3] = {};
+      if (valid) {
+        const RowKet &kt = a.ket[j];
+        koff = kt.pp_off;
+        nkp = kt.npp;
+        c = kt.colc;
+        d = kt.cold;
+        fc = kt.bfc;
+        fd = kt.bfd;
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          Cc[e] = kt.C[e];
+          CD[e] = kt.CD[e];
+        }
+      }
+      R I[K::NC];
+#pragma unroll
+      for (int o = 0; o < K::NC; ++o) I[o] = 0;
+      eval_bra<LA, LB, LC, LD, R>(a.prims, a.primc32, s_tab, bp, Cc, CD, koff, nkp, g, G, I);
+      for (int off = G >> 1; off > 0; off >>= 1) {
+#pragma unroll
+        for (int o = 0; o < K::NC; ++o) I[o] += __shfl_xor(I[o], off);
+      }
+      const bool take = valid && g == 0;
+      // degeneracy in the 8-fold loop (direct.hpp:1664-1667, 1793-1802) and the 1/2 of :1849-1850
+      const double scale =
+          take ? bra_scale * (LC == LD && c == d ? 1.0 : 2.0) * (a.same_class && i == j ? 1.0 : 2.0) : 0.0;
+      double Id[K::NC];
+#pragma unroll
+      for (int o = 0; o < K::NC; ++o) Id[o] = (double)I[o] * scale;
+      if (take)
+        for (int p = 0; p < a.nk; ++p) {
+          const RowPlane &rp = a.k[p];
+          if (!((mask >> rp.mat) & 1u)) continue;
+          if constexpr (XL) {
+            const double *xs = s_x + p * NROW * w;
+            digest_rows<K>(Id, [&](int r, int e, bool second) { return xs[r * w + (second ? d : c) + e]; },
+                           s_k + p * NROW * w, w, c, d);
+          } else {
+            const GlobalDouble *x = (const GlobalDouble *)(one ? a.m0.kx[rp.kind] : mp->kx[rp.kind]) + rp.idx;
+            const int S = a.kps[rp.kind];
+            digest_rows<K>(
+                Id,
+                [&](int r, int e, bool second) {
+                  const unsigned f = (second ? fd : fc) + e, fr = r < K::NCA ? bfa + r : bfb + (r - K::NCA);
+                  return rp.sign * x[(size_t)(rp.colwise ? f + fr * N : fr + f * N) * S];
+                },
+                s_k + p * NROW * w, w, c, d);
+          }
+        }
+      for (int p = 0; p < a.nj; ++p) {
+        // J(a, b) += I X(d, c) over the wave, J(d, c) += I X(a, b) (direct.hpp:1863-1883, 1925-1960)
+        const bool on = take && ((mask >> a.jmat[p]) & 1u);
+        double x[NCD];
+#pragma unroll
+        for (int e = 0; e < NCD; ++e) x[e] = on ? a.jx_ket[(size_t)(p * NCD + e) * a.nket + j] : 0.0;
+        double t[NCD];
+#pragma unroll
+        for (int e = 0; e < NCD; ++e) t[e] = 0.0;
+#pragma unroll
+        for (int ab = 0; ab < NAB; ++ab) {
+          const double xab = as_const(a.jx_bra)[(size_t)(p * NAB + ab) * a.nbra + i];
+          double s = 0.0;
+#pragma unroll
+          for (int e = 0; e < NCD; ++e) {
+            s = fma(Id[ab * NCD + e], x[e], s);
+            t[e] = fma(Id[ab * NCD + e], xab, t[e]);
+          }
+          s = wave_sum(s);
+          if (lane == 0) unsafeAtomicAdd(&s_jab[p * NAB + ab], s);
+        }
+        if (on)
+#pragma unroll
+          for (int e = 0; e < NCD; ++e)
+            unsafeAtomicAdd(a.ja_ket + (size_t)(p * NCD + e) * a.nket + j, a.jcoef[p] * t[e]);
+      }
+    }
+    __syncthreads();
+    // rows and J(a, b) out
+    for (int p = 0; p < a.nk; ++p) {
+      const RowPlane &rp = a.k[p];
+      GlobalDouble *acc = (GlobalDouble *)(one ? a.m0.ka[rp.kind] : mp->ka[rp.kind]) + rp.idx;
+      const int S = a.kps[rp.kind];
+      const double *ks = s_k + p * NROW * w;
+      const double coef = 0.5 * rp.sign;
+      for (int c = tid; c < w; c += kRowThreads) {
+        const int f = colmap[c];
+        if (f < 0) continue;
+#pragma unroll
+        for (int r = 0; r < NROW; ++r) {
+          const int fr = r < K::NCA ? bfa + r : bfb + (r - K::NCA);
+          const double v = ks[r * w + c];
+          if (v != 0.0)
+            __builtin_amdgcn_global_atomic_fadd_f64(
+                acc + (size_t)(rp.colwise ? f + (size_t)fr * N : fr + (size_t)f * N) * S, coef * v);
+        }
+      }
+    }
+    for (int e = tid; e < a.nj * NAB; e += kRowThreads) {
+      const double v = s_jab[e];
+      if (v != 0.0) unsafeAtomicAdd(a.ja_bra + (size_t)e * a.nbra + i, a.jcoef[e / NAB] * v);
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    if (s_tot[0]) atomicAdd(a.count, s_tot[0]);
+    if (s_tot[1]) atomicAdd(a.count + 1, s_tot[1]);
+    if (s_psum != 0.0) unsafeAtomicAdd(a.prim_sum, s_psum);
+  }
+}
+
+// LDS of a block in bytes: the static arrays (with padding) and sets sets of
+// rows (exchange, and density)
+template <class K, class R>
+size_t row_lds(int nk, int width, int sets) {
+  const size_t fixed = sizeof(R) * rys_tab_len(K::NR) + 4 * kRowChunk + 8 * kRowJ * K::NCA * K::NCB + 256;
+  return fixed + (size_t)sets * nk * (K::NCA + K::NCB) * width * sizeof(double);
+}
+
+constexpr size_t kRowLdsMax = 160 * 1024;
+constexpr long long kRowGrid = 8192;
+
+template <int LA, int LB, int LC, int LD, class R, bool XL>
+hipError_t launch_row_x(const RowLaunch &a, hipStream_t s) {
+  using K = Cls<LA, LB, LC, LD>;
+  auto kern = eri_row_kernel<LA, LB, LC, LD, R, XL>;
+  static std::once_flag once;  // allow dynamic LDS beyond the default limit, once per instantiation
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [&] {
+    attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               160 * 1024 - (int)row_lds<K, R>(0, 0, 0));
+  });
+  if (attr != hipSuccess) return attr;
+  const long long items = (long long)a.nbra * a.nchunk;
+  const size_t dyn = (size_t)(XL ? 2 : 1) * a.nk * (K::NCA + K::NCB) * a.width * sizeof(double);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(items < kRowGrid ? items : kRowGrid)), dim3(row_threads<K>()), dyn, s, a);
+  return hipGetLastError();
+}
+
+template <int LA, int LB, int LC, int LD, class R>
+hipError_t launch_row_cls(const RowLaunch &a, hipStream_t s) {
+  using K = Cls<LA, LB, LC, LD>;
+  if ((long long)a.nbra * a.nchunk <= 0) return hipSuccess;
+  // density rows in LDS where both sets fit: GHF (H2O)16 (eight planes)
+  // takes the second form for (ps|ps) and up, 11.5 -> 9.4 ms a build with it
+  if (row_lds<K, R>(a.nk, a.width, 2) <= kRowLdsMax) return launch_row_x<LA, LB, LC, LD, R, true>(a, s);
+  if (row_lds<K, R>(a.nk, a.width, 1) <= kRowLdsMax) return launch_row_x<LA, LB, LC, LD, R, false>(a, s);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+// classes with a row kernel, in three groups that compile apart
+#define CQX_ROW_CLASSES_A(X) X(0, 0, 0, 0) X(1, 0, 0, 0) X(1, 0, 1, 0) X(1, 1, 0, 0) X(2, 0, 0, 0) X(1, 1, 1, 0)
+#define CQX_ROW_CLASSES_B(X) X(2, 0, 1, 0) X(2, 1, 0, 0) X(2, 0, 2, 0) X(2, 2, 0, 0) X(2, 1, 1, 0)
+#define CQX_ROW_CLASSES_C(X) X(2, 0, 1, 1) X(1, 1, 1, 1) X(2, 1, 2, 0) X(2, 2, 1, 0)
+
+template <int GROUP>
+hipError_t launch_row_group(const RowLaunch &a, hipStream_t s);
+template <int GROUP>
+bool row_group_lds(int la, int lb, int lc, int ld, int fp32, int nk, int width, size_t &bytes);
+
+#define CQX_ROW_GROUP(GROUP, LIST)                                                                         \
+  template <>                                                                                              \
+  hipError_t launch_row_group<GROUP>(const RowLaunch &a, hipStream_t s) {                                  \
+    LIST(CQX_ROW_LAUNCH) return hipErrorNotSupported;                                                      \
+  }                                                                                                        \
+  template <>                                                                                              \
+  bool row_group_lds<GROUP>(int la, int lb, int lc, int ld, int fp32, int nk, int width, size_t &bytes) {  \
+    LIST(CQX_ROW_LDS) return false;                                                                        \
+  }
+#define CQX_ROW_LAUNCH(A, B, C, D)                          \
+  if (a.la == A && a.lb == B && a.lc == C && a.ld == D)     \
+    return a.fp32 ? launch_row_cls<A, B, C, D, float>(a, s) \
+                  : launch_row_cls<A, B, C, D, double>(a, s);
+#define CQX_ROW_LDS(A, B, C, D)                                             \
+  if (la == A && lb == B && lc == C && ld == D) {                           \
+    bytes = fp32 ? row_lds<Cls<A, B, C, D>, float>(nk, width, 1)               \
+                 : row_lds<Cls<A, B, C, D>, double>(nk, width, 1);             \
+    return true;                                                            \
+  }
+
+}  // namespace cqx

@@ -17,7 +17,10 @@
 #include <hip/hip_runtime.h>
 
 #include "digest.hpp"
-#include "eri_fast_impl.hpp"
+#include "digest_tile.hpp"
+#include "eri_class.hpp"
+#include "kernels.hpp"
+#include "limits.hpp"
 
 namespace cqx {
 
@@ -164,8 +167,8 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void eri_wave_kernel(EriLaunch
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
           PQ[d] = A.P[d] - B.P[d];
-          PAv[d] = A.PA[d];
-          QCv[d] = B.PA[d];
+          PAv[d] = A.P[d] - bp.A[d];
+          QCv[d] = B.P[d] - kp.A[d];
         }
       }
       const PrimRecip<R> pr = prim_recip<R>(ap, bq, kk);

@@ -156,7 +156,7 @@ __global__ __launch_bounds__(64) void eri_grad_kernel(GradLaunch a) {
         __syncthreads();
         if (lane < 3 * nrp) {
           const int lr = lane / 3, dir = lane % 3, r = r0 + lr;
-          rys_2d_grad(D, s_x[r], A.p, B.p, A.PA[dir], B.PA[dir], PQ[dir], bp.AB[dir], kp.AB[dir],
+          rys_2d_grad(D, s_x[r], A.p, B.p, A.P[dir] - bp.A[dir], B.P[dir] - kp.A[dir], PQ[dir], bp.AB[dir], kp.AB[dir],
                       dir == 2 ? s_w[r] : 1.0, s_H + (size_t)(lr * 3 + dir) * D.nh);
         }
         __syncthreads();

@@ -17,6 +17,7 @@
 #include "digest.hpp"
 #include "kernels.hpp"
 #include "rys.hpp"
+#include "screen.hpp"
 
 namespace cqx {
 
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(64) void eri_team_kernel(EriLaunch a) {
             __syncthreads();
             if (lane < 3 * nrp) {
               const int lr = lane / 3, dir = lane % 3, r = r0 + lr;
-              rys_2d(D, s_x[r], A.p, B.p, A.PA[dir], B.PA[dir], PQ[dir], bp.AB[dir], kp.AB[dir],
+              rys_2d(D, s_x[r], A.p, B.p, A.P[dir] - bp.A[dir], B.P[dir] - kp.A[dir], PQ[dir], bp.AB[dir], kp.AB[dir],
                      dir == 2 ? s_w[r] : 1.0, s_H + (lr * 3 + dir) * D.nh);
             }
             __syncthreads();
@@ -215,65 +216,6 @@ __global__ __launch_bounds__(64) void eri_team_kernel(EriLaunch a) {
 // of contractions that pass their own separated screen.
 // ---------------------------------------------------------------------------
 constexpr int kListThreads = 1024;
-
-// The reference's screen of one candidate quartet (bra pair P with its own
-// block norms pb, ket pair Q with pk): the Schwarz product against the max
-// of the six shell-block norms in reference labels (the pair the reference
-// loop visits later is the bra), globally and per matrix (separated
-// screen).  Returns whether any contraction survives and their mask.
-struct ScreenArgs {
-  const double *Bg, *Bm;
-  const long long *mol_boff;
-  const int *mol_ns;
-  int nmat;
-  double thresh;
-  int screen;
-};
-__device__ __forceinline__ bool screen_candidate(const ScreenArgs &a, const PairScr &P, const PairScr &Q,
-                                                 const double *pb, const double *pk, double qq, unsigned &mask) {
-  mask = 0;
-  const int ps1 = (int)(P.s12 & 0xFFFFu), ps2 = (int)(P.s12 >> 16);
-  const int qs1 = (int)(Q.s12 & 0xFFFFu), qs2 = (int)(Q.s12 >> 16);
-  const bool p_first = (ps1 > qs1) || (ps1 == qs1 && ps2 >= qs2);
-  const int s1 = p_first ? ps1 : qs1, s2 = p_first ? ps2 : qs2;
-  const int s3 = p_first ? qs1 : ps1, s4 = p_first ? qs2 : ps2;
-  // lower bounds from the pairs' own block norms: enough to accept
-  if (!a.screen) {
-    mask = (1u << a.nmat) - 1u;
-    return true;
-  }
-  if (!(fmax(pb[0], pk[0]) * qq < a.thresh)) {
-    if (a.nmat == 1) {
-      mask = 1u;
-      return true;
-    }
-    unsigned lm = 0;
-    for (int m = 0; m < a.nmat; ++m)
-      if (!(fmax(pb[1 + m], pk[1 + m]) * qq < a.thresh)) lm |= 1u << m;
-    if (lm == (1u << a.nmat) - 1u) {
-      mask = lm;
-      return true;
-    }
-  }
-  const long long boff = a.mol_boff[P.mol];
-  const int ns = a.mol_ns[P.mol];
-  auto bmax = [&](const double *B, int ld, int m) {
-    auto at = [&](int x, int y) { return B[(boff + x + (size_t)y * ns) * ld + m]; };
-    double v = fmax(at(s1, s2), fmax(at(s1, s3), at(s2, s3)));
-    v = fmax(v, at(s3, s4));
-    v = fmax(v, fmax(at(s1, s4), at(s2, s4)));
-    return v;
-  };
-  if (bmax(a.Bg, 1, 0) * qq < a.thresh) return false;
-  if (a.nmat == 1) {
-    mask = 1u;
-  } else {
-    // per-matrix norms interleaved: the nmat values of one block share a line
-    for (int m = 0; m < a.nmat; ++m)
-      if (!(bmax(a.Bm, a.nmat, m) * qq < a.thresh)) mask |= 1u << m;
-  }
-  return mask != 0u;
-}
 
 // Candidates [base, base + 1024) of one list: the block's bra range is found
 // once, each thread tests one candidate, survivors are appended block-wide

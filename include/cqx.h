@@ -258,7 +258,12 @@ int cqx_grad_two_body_contract(cqx_ctx *ctx, int ngrad, int nmat, const cqx_cont
  * of (ss|ss), (ps|ss), (ps|ps), (pp|ss), (pp|ps), (ds|ss), (ds|ps), (dp|ss)
  * takes tiles; default 126, all but (ss|ss) and (dp|ss)), "rys_lds" (1, the
  * default: the lane-group kernels read the Rys table section of their root
- * count from a copy in LDS; 0: from global memory).  Setting any option
+ * count from a copy in LDS; 0: from global memory), "rows" (1, the default:
+ * a class pair with a row kernel, whose rows of the build's exchange planes
+ * fit in LDS, screens, evaluates and digests its quartets in one launch
+ * without quartet lists; 0: quartet lists for every class pair;
+ * allocation-free builds, and builds with "fast_lanes" set, always take
+ * lists).  Setting any option
  * drops a recorded graph. */
 int cqx_set_option(cqx_ctx *ctx, const char *name, double value);
 
