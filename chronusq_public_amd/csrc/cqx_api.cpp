@@ -294,6 +294,30 @@ void drop_graph(cqx_ctx *c) {
   c->graph_key.clear();
 }
 
+// Side streams for concurrent class-pair launches: created outside any
+// capture, forked from the context stream before the launches and joined
+// back into it after them (also inside a recorded build); the
+// allocation-free path launches on the context stream alone.
+void ensure_sides(cqx_ctx *c, int nst) {
+  for (int i = 0; i < nst - 1; ++i)
+    if (!c->side[i]) {
+      HIPCHK(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
+      HIPCHK(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
+    }
+  if (nst > 1 && !c->ev_fork) HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+}
+void fork_sides(cqx_ctx *c, int nst) {
+  if (nst <= 1) return;
+  HIPCHK(hipEventRecord(c->ev_fork, c->stream));
+  for (int i = 0; i < nst - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
+}
+void join_sides(cqx_ctx *c, int nst) {
+  for (int i = 0; i < nst - 1; ++i) {
+    HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
+    HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join[i], 0));
+  }
+}
+
 // contraction signature: what the recorded launches depend on besides the
 // densities themselves
 std::string contraction_key(int screen, int is_complex, int ncon, const cqx_contraction *list) {
@@ -1681,29 +1705,9 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       front();
       const bool mixed = c->fp32_cut > 0.0;
       const int qmul = mixed ? 2 : 1;  // quartet lists per class pair
-      // side streams for concurrent class-pair launches: created outside any
-      // capture, forked from the context stream before the launches and
-      // joined back into it after them (also inside a recorded build); the
-      // allocation-free path launches on the context stream alone
-      auto ensure_side = [&](int nst) {
-        for (int i = 0; i < nst - 1; ++i)
-          if (!c->side[i]) {
-            HIPCHK(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
-            HIPCHK(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
-          }
-        if (nst > 1 && !c->ev_fork) HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-      };
-      auto fork_side = [&](int nst) {
-        if (nst <= 1) return;
-        HIPCHK(hipEventRecord(c->ev_fork, s));
-        for (int i = 0; i < nst - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
-      };
-      auto join_side = [&](int nst) {
-        for (int i = 0; i < nst - 1; ++i) {
-          HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
-          HIPCHK(hipStreamWaitEvent(s, c->ev_join[i], 0));
-        }
-      };
+      auto ensure_side = [&](int nst) { ensure_sides(c, nst); };
+      auto fork_side = [&](int nst) { fork_sides(c, nst); };
+      auto join_side = [&](int nst) { join_sides(c, nst); };
       auto stream_of = [&](int launch, int nst) { return launch % nst == 0 ? s : c->side[launch % nst - 1]; };
       const bool tuning = c->autotune_pending && !scr;  // the allocation-free path never times
       const int nst_all = (tuning || scr) ? 1 : c->nstreams;
@@ -2673,8 +2677,13 @@ int cqx_grad_two_body_contract(cqx_ctx *c, int ngrad, int nmat, const cqx_contra
     const size_t nacc = (size_t)ngrad * nmat * nbc2;
     c->d_gacc.ensure(nacc);
     HIPCHK(cqx::launch_zero(c->d_gacc.p, nacc, s));
-    // every quartet of every class pair (bra class >= ket class)
+    // every quartet of every class pair (bra class >= ket class), dealt over
+    // the launch streams: the higher classes have few quartets
+    const int nst = c->nstreams;
+    int nlaunched = 0;
+    ensure_sides(c, nst);
     HIPCHK(hipEventRecord(c->ev0, s));
+    fork_sides(c, nst);
     for (int cb = 0; cb < kNumClass; ++cb)
       for (int ck = 0; ck <= cb; ++ck) {
         const long long nbra = (long long)c->cls[cb].size(), nket = (long long)c->cls[ck].size();
@@ -2700,19 +2709,20 @@ int cqx_grad_two_body_contract(cqx_ctx *c, int ngrad, int nmat, const cqx_contra
         G.nmat = nmat;
         G.nbc = nbc;
         G.kmask = kmask;
-        HIPCHK(cqx::launch_eri_grad(G, s));
+        HIPCHK(cqx::launch_eri_grad(G, nlaunched % nst == 0 ? s : c->side[nlaunched % nst - 1]));
+        ++nlaunched;
         c->stats.n_quartets += G.nq;
         c->stats.n_launch_eri++;
       }
+    join_sides(c, nst);
     HIPCHK(hipEventRecord(c->ev1, s));
     // back to pure functions, Hermitian symmetrisation into AX
     // (AX += 1/2 (A + A^T), direct.hpp:2548-2570), per coordinate and matrix
     const size_t nout = (size_t)ngrad * nmat;
     c->d_gAX.ensure(nout * nb2);
-    for (size_t k = 0; k < nout; ++k) {
+    for (size_t k = 0; k < nout; ++k)
       HIPCHK(hipMemcpyAsync(c->d_gAX.p + k * nb2, list[k].AX, sizeof(double) * nb2, hk, s));
-      HIPCHK(cqx::launch_from_cart(c->cmap, c->d_gacc.p + k * nbc2, nullptr, 1, 1, 0, c->d_gAX.p + k * nb2, s));
-    }
+    HIPCHK(cqx::launch_from_cart_many(c->cmap, c->d_gacc.p, nbc2, 1, c->d_gAX.p, nb2, nout, s));
     const hipMemcpyKind dk = mem == CQX_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     for (size_t k = 0; k < nout; ++k)
       HIPCHK(hipMemcpyAsync(list[k].AX, c->d_gAX.p + k * nb2, sizeof(double) * nb2, dk, s));

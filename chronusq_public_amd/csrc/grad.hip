@@ -1,6 +1,8 @@
 // Nuclear-gradient J/K contraction: the derivative integrals of every
 // shell quartet digested into one J or K matrix per nuclear coordinate,
-// DirectGradContraction::directScaffoldGrad (direct.hpp:2198-2580).
+// DirectGradContraction::directScaffoldGrad (direct.hpp:2198-2580).  The
+// s/p/d classes have templated kernels (eri_grad_impl.hpp); this is the
+// generic one.
 //
 // One 64-lane wave per shell quartet, any class through (gg|gg).  Per primitive
 // quartet the Rys 2D integrals are built with one more unit of angular
@@ -275,8 +277,20 @@ int grad_chunk(int la, int lb, int lc, int ld, size_t lds_max, int *rpp_out) {
   return best;
 }
 
+template <int GROUP>
+hipError_t launch_grad_group(const GradLaunch &a, hipStream_t s);
+
+// the templated kernels of the s/p/d classes (eri_grad_impl.hpp), else the
+// generic one
 hipError_t launch_eri_grad(const GradLaunch &a, hipStream_t s) {
   if (a.nq <= 0) return hipSuccess;
+  {
+    hipError_t e = launch_grad_group<0>(a, s);
+    if (e == hipErrorNotSupported) e = launch_grad_group<1>(a, s);
+    if (e == hipErrorNotSupported) e = launch_grad_group<2>(a, s);
+    if (e == hipErrorNotSupported) e = launch_grad_group<3>(a, s);
+    if (e != hipErrorNotSupported) return e;
+  }
   if (a.la > kMaxLDev || a.lb > kMaxLDev || a.lc > kMaxLDev || a.ld > kMaxLDev || a.chunk <= 0 || a.rpp <= 0)
     return hipErrorNotSupported;
   const int nc = ((a.la + 1) * (a.la + 2) / 2) * ((a.lb + 1) * (a.lb + 2) / 2) * ((a.lc + 1) * (a.lc + 2) / 2) *

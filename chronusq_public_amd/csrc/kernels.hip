@@ -548,8 +548,11 @@ __global__ void to_cart_kernel(CartMap M, const double *X, int cplx, double *Pre
   if (Pim) Pim[t * ps] = im;
 }
 
+// blockIdx.y: matrix of a batch of equal ones, sa / sx doubles apart
 __global__ void from_cart_kernel(CartMap M, const double *Are, const double *Aim, int ps,
-                                 int her, int cplx, double *AX) {
+                                 int her, int cplx, double *AX, size_t sa, size_t sx) {
+  Are += blockIdx.y * sa;
+  AX += blockIdx.y * sx;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long long)M.nb * M.nb) return;
   const int mu = (int)(t % M.nb), nu = (int)(t / M.nb);
@@ -710,7 +713,17 @@ hipError_t launch_to_cart(const CartMap &m, const double *X, int is_complex, dou
 hipError_t launch_from_cart(const CartMap &m, const double *are, const double *aim, int ps, int her,
                             int is_complex, double *AX, hipStream_t s) {
   hipLaunchKernelGGL(from_cart_kernel, dim3(nblocks((long long)m.nb * m.nb, 256)), dim3(256), 0,
-                     s, m, are, aim, ps, her, is_complex, AX);
+                     s, m, are, aim, ps, her, is_complex, AX, (size_t)0, (size_t)0);
+  return hipGetLastError();
+}
+
+hipError_t launch_from_cart_many(const CartMap &m, const double *a, size_t sa, int her, double *AX, size_t sx,
+                                 size_t n, hipStream_t s) {
+  for (size_t k = 0; k < n; k += 65535) {
+    const unsigned ny = (unsigned)std::min<size_t>(65535, n - k);
+    hipLaunchKernelGGL(from_cart_kernel, dim3(nblocks((long long)m.nb * m.nb, 256), ny), dim3(256), 0, s, m, a + k * sa,
+                       (const double *)nullptr, 1, her, 0, AX + k * sx, sa, sx);
+  }
   return hipGetLastError();
 }
 

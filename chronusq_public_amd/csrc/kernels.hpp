@@ -251,6 +251,9 @@ hipError_t launch_to_cart(const CartMap &m, const double *X, int is_complex,
 // A_im may be null (real accumulator only); planes interleaved with stride ps.
 hipError_t launch_from_cart(const CartMap &m, const double *A_re, const double *A_im, int ps,
                             int her, int is_complex, double *AX, hipStream_t s);
+// n real matrices, sa / sx doubles apart, in one launch
+hipError_t launch_from_cart_many(const CartMap &m, const double *a, size_t sa, int her, double *AX, size_t sx,
+                                 size_t n, hipStream_t s);
 
 hipError_t launch_zero(double *p, size_t n, hipStream_t s);
 

@@ -93,10 +93,11 @@ __device__ __forceinline__ void rys_roots(R T, const R *__restrict__ tab, R *__r
   }
 }
 
-// Root r (and its weight) of an N-point rule, N known at compile time.
+// Root r (and its weight) of an N-point rule, N known at compile time; tabn
+// points at the table's N-root section.
 template <int N, class R>
-__device__ __forceinline__ void rys_root(R T, const R *__restrict__ tab, int r, R &x, R &w) {
-  constexpr int kTcut = 34 + 6 * N, kOff = rys_tab_off(N);
+__device__ __forceinline__ void rys_root_sec(R T, const R *__restrict__ tabn, int r, R &x, R &w) {
+  constexpr int kTcut = 34 + 6 * N;
   if (T >= (R)kTcut) {
     const R rt = eval_rcp<R>(T);
     x = (R)cqx_rys_asym_x[N][r] * rt;
@@ -104,10 +105,15 @@ __device__ __forceinline__ void rys_root(R T, const R *__restrict__ tab, int r, 
   } else {
     const int i = (int)T;
     const R u = (R)2 * (T - (R)i) - (R)1;
-    const R *c = tab + kOff + (size_t)i * (2 * N * CQX_RYS_NCOEF);
+    const R *c = tabn + (size_t)i * (2 * N * CQX_RYS_NCOEF);
     x = chebyshev<R>(c + r * CQX_RYS_NCOEF, u);
     w = chebyshev<R>(c + (N + r) * CQX_RYS_NCOEF, u);
   }
+}
+// the same from the whole table
+template <int N, class R>
+__device__ __forceinline__ void rys_root(R T, const R *__restrict__ tab, int r, R &x, R &w) {
+  rys_root_sec<N, R>(T, tab + rys_tab_off(N), r, x, w);
 }
 
 // Root r (and its weight) of an n-point rule, n (<= CQX_RYS_NMAX) known at
