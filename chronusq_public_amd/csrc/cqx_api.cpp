@@ -1768,6 +1768,8 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             cqx::RowLaunch R = row0;
             class_ls(cb, R.la, R.lb);
             class_ls(ck, R.lc, R.ld);
+            const bool split = mixed && R.la <= 2;  // f and g classes stay in FP64
+            if (f && !split) continue;
             R.bra = c->d_pairs[cb].p;
             R.bscr = c->d_scr[cb].p;
             R.kscr = c->d_scr[ck].p;
@@ -1789,7 +1791,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             R.nmat = nmat;
             R.thresh = c->thresh;
             R.screen = screen;
-            R.cut32 = mixed ? c->fp32_cut : 0.0;
+            R.cut32 = split ? c->fp32_cut : 0.0;
             R.fp32 = f;
             R.prims = c->d_prims.p;
             R.primc32 = c->d_primc32.p;

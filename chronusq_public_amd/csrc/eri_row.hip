@@ -16,7 +16,8 @@ namespace {
 bool row_lds_of(int la, int lb, int lc, int ld, int fp32, int nk, int width, size_t &bytes) {
   return row_group_lds<0>(la, lb, lc, ld, fp32, nk, width, bytes) ||
          row_group_lds<1>(la, lb, lc, ld, fp32, nk, width, bytes) ||
-         row_group_lds<2>(la, lb, lc, ld, fp32, nk, width, bytes);
+         row_group_lds<2>(la, lb, lc, ld, fp32, nk, width, bytes) ||
+         row_group_lds<3>(la, lb, lc, ld, fp32, nk, width, bytes);
 }
 
 __device__ __forceinline__ const MolPlanes &planes_of(const PairOrder &a, int mol) {
@@ -71,6 +72,7 @@ hipError_t launch_eri_row(const RowLaunch &a, hipStream_t s) {
   hipError_t e = launch_row_group<0>(a, s);
   if (e == hipErrorNotSupported) e = launch_row_group<1>(a, s);
   if (e == hipErrorNotSupported) e = launch_row_group<2>(a, s);
+  if (e == hipErrorNotSupported) e = launch_row_group<3>(a, s);
   return e;
 }
 

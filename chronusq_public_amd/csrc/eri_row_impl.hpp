@@ -438,12 +438,24 @@ hipError_t launch_row_cls(const RowLaunch &a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
+template <int LA, int LB, int LC, int LD>
+hipError_t launch_row_prec(const RowLaunch &a, hipStream_t s) {
+  if (!a.fp32) return launch_row_cls<LA, LB, LC, LD, double>(a, s);
+  if constexpr (LA <= 2) return launch_row_cls<LA, LB, LC, LD, float>(a, s);
+  return hipErrorInvalidValue;
+}
+
 }  // namespace
 
-// classes with a row kernel, in three groups that compile apart
+// classes with a row kernel, in groups that compile apart
 #define CQX_ROW_CLASSES_A(X) X(0, 0, 0, 0) X(1, 0, 0, 0) X(1, 0, 1, 0) X(1, 1, 0, 0) X(2, 0, 0, 0) X(1, 1, 1, 0)
 #define CQX_ROW_CLASSES_B(X) X(2, 0, 1, 0) X(2, 1, 0, 0) X(2, 0, 2, 0) X(2, 2, 0, 0) X(2, 1, 1, 0)
 #define CQX_ROW_CLASSES_C(X) X(2, 0, 1, 1) X(1, 1, 1, 1) X(2, 1, 2, 0) X(2, 2, 1, 0)
+// with an f or g shell, up to 45 components (FP64 only, as their quartet
+// lists): (fs|ss) of (H2O)6 / cc-pVTZ 0.61 ms on the wave kernel, 0.21 here,
+// but (fs|ds) 0.25 and 0.60: beyond, a block holds one wave per SIMD
+#define CQX_ROW_CLASSES_D(X) \
+  X(3, 0, 0, 0) X(3, 0, 1, 0) X(3, 1, 0, 0) X(4, 0, 0, 0) X(4, 0, 1, 0) X(4, 1, 0, 0)
 
 template <int GROUP>
 hipError_t launch_row_group(const RowLaunch &a, hipStream_t s);
@@ -461,8 +473,7 @@ bool row_group_lds(int la, int lb, int lc, int ld, int fp32, int nk, int width, 
   }
 #define CQX_ROW_LAUNCH(A, B, C, D)                          \
   if (a.la == A && a.lb == B && a.lc == C && a.ld == D)     \
-    return a.fp32 ? launch_row_cls<A, B, C, D, float>(a, s) \
-                  : launch_row_cls<A, B, C, D, double>(a, s);
+    return launch_row_prec<A, B, C, D>(a, s);
 #define CQX_ROW_LDS(A, B, C, D)                                             \
   if (la == A && lb == B && lc == C && ld == D) {                           \
     bytes = fp32 ? row_lds<Cls<A, B, C, D>, float>(nk, width, 1)               \

@@ -17,7 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include "digest.hpp"
-#include "digest_tile.hpp"
+#include "digest_staged.hpp"
 #include "eri_class.hpp"
 #include "kernels.hpp"
 #include "limits.hpp"
@@ -48,10 +48,21 @@ constexpr int wave_buf_doubles() {
   return tables > QT * K::NC ? tables : QT * K::NC;
 }
 
+// A wave's staged density elements in doubles: those of its QT quartets for
+// a real J/K pair, at least of one, within 512.  Staged above 216
+// components only: (fp|dp) and (fd|dp) of (H2O)6 / cc-pVTZ 0.83 -> 0.64 and
+// 0.68 -> 0.59 ms, but (fd|ps) 0.23 -> 0.27 and (fs|dp) 0.225 -> 0.244 (the
+// LDS costs a block per CU).
+template <class K, int QT>
+constexpr int wave_xcap() {
+  constexpr int one = XLayout<K>::EJ + XLayout<K>::EK;
+  return K::NC <= 216 ? 0 : one * QT <= 512 ? one * QT : one > 512 ? one : 512;
+}
+
 // LDS of a block of the kernel below with QT quartets per wave
 template <class K, class R, int QT>
 constexpr int wave_lds_bytes() {
-  return kWavesPerBlock * (wave_buf_doubles<K, R, QT>() * 8 + QT * 24 + QT * 2 * (int)sizeof(PairRec));
+  return kWavesPerBlock * (8 * wave_xcap<K, QT>() + wave_buf_doubles<K, R, QT>() * 8 + QT * 24 + QT * 2 * (int)sizeof(PairRec));
 }
 
 // QT: quartets a wave takes together.  Their primitive quartets form one
@@ -68,6 +79,8 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void eri_wave_kernel(EriLaunch
   constexpr int HSZ = 3 * K::NR * K::NH;
   constexpr int PP = prims_per_round<K, R>();
   __shared__ double s_buf[kWavesPerBlock][wave_buf_doubles<K, R, QT>()];
+  constexpr int XCAP = wave_xcap<K, QT>();
+  __shared__ double s_X[kWavesPerBlock][XCAP > 0 ? XCAP : 1];
   __shared__ int s_bf[kWavesPerBlock][QT][4];
   __shared__ unsigned s_mask[kWavesPerBlock][QT];
   __shared__ int s_mol[kWavesPerBlock][QT];
@@ -229,7 +242,10 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void eri_wave_kernel(EriLaunch
       if (lane + 64 * k < K::NC) sI[t * K::NC + lane + 64 * k] = (double)acc[t][k] * scale;
   }
   wave_sync();
-  digest_tile<K>(sI, s_bf[wv], s_mask[wv], s_mol[wv], ntile, a.planes, lane);
+  if constexpr (XCAP > 0)
+    digest_staged<K, XCAP>(sI, s_bf[wv], s_mask[wv], s_mol[wv], ntile, a.planes, s_X[wv], lane);
+  else
+    digest_tile<K>(sI, s_bf[wv], s_mask[wv], s_mol[wv], ntile, a.planes, lane);
 }
 
 // LDS a block may take on gfx950 (160 KB per CU): variants beyond it are

@@ -1,6 +1,6 @@
 // HIP kernels of the direct J/K build for gfx950 (MI355X): screening and
-// quartet-list construction, the generic Rys ERI + digestion kernel, and the
-// matrix transforms around them.
+// quartet-list construction, and the matrix transforms around the ERI
+// kernels.
 //
 // Reference algorithm: GTODirectTPIContraction::directScaffoldNew
 // (include/particleintegrals/contract/direct.hpp:1412-2123).  The quartet set,
@@ -12,202 +12,17 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <mutex>
 
-#include "digest.hpp"
 #include "kernels.hpp"
-#include "rys.hpp"
 #include "screen.hpp"
 
 namespace cqx {
 
 namespace {
 
-constexpr double kTwoPi52 = 34.98683665524972;  // 2 pi^(5/2)
-
 __device__ __forceinline__ int ncart_d(int l) { return (l + 1) * (l + 2) / 2; }
 
-// Cartesian exponents of component c of an l shell (lx descending, then ly).
-__device__ __forceinline__ void cart_exp(int l, int c, int &lx, int &ly, int &lz) {
-  int k = c;
-  lx = l;
-  while (k >= l - lx + 1) {
-    k -= l - lx + 1;
-    --lx;
-  }
-  lz = k;
-  ly = l - lx - lz;
-}
-
 __device__ __forceinline__ void atomic_add(double *p, double v) { unsafeAtomicAdd(p, v); }
-
-// ---------------------------------------------------------------------------
-// Generic Rys ERI kernel: one 64-lane wave per shell quartet.
-// Per primitive quartet, lanes r < NR fetch the Rys nodes/weights, lanes
-// (r, dir) < 3 NR build the 2D integrals I_dir(ia, ib, ic, id) (vertical
-// recursion on the Rys variables, then horizontal transfer to b and d) into
-// LDS, and every lane accumulates its share of the Cartesian quartet in LDS.
-// Quartets too large for LDS (classes with g shells) are built in passes
-// over ranges of the first shell's components (a is the slowest index of
-// the quartet layout, so a range is a smaller quartet with a's first
-// function shifted) and with the 2D tables of a few roots at a time; each
-// pass is digested (or stored) on its own, since every J/K update is a sum
-// of terms linear in the integrals.
-// ---------------------------------------------------------------------------
-struct TeamDims {
-  int la, lb, lc, ld, nca, ncb, ncc, ncd, nc, ni, nk, nr, nh;
-};
-
-__device__ TeamDims team_dims(int la, int lb, int lc, int ld) {
-  TeamDims d;
-  d.la = la; d.lb = lb; d.lc = lc; d.ld = ld;
-  d.nca = ncart_d(la); d.ncb = ncart_d(lb); d.ncc = ncart_d(lc); d.ncd = ncart_d(ld);
-  d.nc = d.nca * d.ncb * d.ncc * d.ncd;
-  d.ni = la + lb + 1;
-  d.nk = lc + ld + 1;
-  d.nr = (la + lb + lc + ld) / 2 + 1;
-  d.nh = (la + 1) * (lb + 1) * (lc + 1) * (ld + 1);
-  return d;
-}
-
-constexpr int kTeamMaxI = 2 * kMaxLDev + 1;  // la + lb + 1
-
-// 2D integrals of one Rys root along one direction, written to H[nh].
-__device__ void rys_2d(const TeamDims &D, double t2, double p, double q, double PAd,
-                       double QCd, double PQd, double ABd, double CDd, double scale,
-                       double *__restrict__ H) {
-  double G[kTeamMaxI][kTeamMaxI];                 // [i <= la+lb][k <= lc+ld]
-  double E[kTeamMaxI][kMaxLDev + 1][kTeamMaxI];   // bra transfer: [i][j][k]
-  const double pq = p + q, rho = p * q / pq;
-  const double B00 = 0.5 * t2 / pq;
-  const double B10 = 0.5 / p * (1.0 - rho / p * t2);
-  const double B01 = 0.5 / q * (1.0 - rho / q * t2);
-  const double C00 = PAd - (q / pq) * t2 * PQd;
-  const double D00 = QCd + (p / pq) * t2 * PQd;
-  G[0][0] = scale;
-  if (D.ni > 1) G[1][0] = C00 * scale;
-  for (int i = 1; i + 1 < D.ni; ++i) G[i + 1][0] = C00 * G[i][0] + i * B10 * G[i - 1][0];
-  for (int k = 0; k + 1 < D.nk; ++k) {
-    G[0][k + 1] = D00 * G[0][k] + (k > 0 ? k * B01 * G[0][k - 1] : 0.0);
-    for (int i = 1; i < D.ni; ++i)
-      G[i][k + 1] = D00 * G[i][k] + (k > 0 ? k * B01 * G[i][k - 1] : 0.0) + i * B00 * G[i - 1][k];
-  }
-  // horizontal transfer on the bra: (i, j+1) = (i+1, j) + AB (i, j)
-  for (int i = 0; i < D.ni; ++i)
-    for (int k = 0; k < D.nk; ++k) E[i][0][k] = G[i][k];
-  for (int j = 1; j <= D.lb; ++j)
-    for (int i = 0; i + j < D.ni; ++i)
-      for (int k = 0; k < D.nk; ++k) E[i][j][k] = E[i + 1][j - 1][k] + ABd * E[i][j - 1][k];
-  // horizontal transfer on the ket for every (ia, ib)
-  for (int ia = 0; ia <= D.la; ++ia)
-    for (int ib = 0; ib <= D.lb; ++ib) {
-      double F[kTeamMaxI][kMaxLDev + 1];
-      for (int k = 0; k < D.nk; ++k) F[k][0] = E[ia][ib][k];
-      for (int l = 1; l <= D.ld; ++l)
-        for (int k = 0; k + l < D.nk; ++k) F[k][l] = F[k + 1][l - 1] + CDd * F[k][l - 1];
-      for (int ic = 0; ic <= D.lc; ++ic)
-        for (int id = 0; id <= D.ld; ++id)
-          H[((ia * (D.lb + 1) + ib) * (D.lc + 1) + ic) * (D.ld + 1) + id] = F[ic][id];
-    }
-}
-
-// LDS of the generic kernel, in doubles: Rys nodes and weights of up to 16
-// roots, the 2D tables of rpp roots and the quartet components of ca
-// components of the first shell
-__host__ __device__ constexpr int team_lds_doubles(int rpp, int nh, int ca, int nbcd) {
-  return 32 + rpp * 3 * nh + ca * nbcd;
-}
-
-__global__ __launch_bounds__(64) void eri_team_kernel(EriLaunch a) {
-  extern __shared__ double lds[];
-  const int lane = threadIdx.x;
-  const TeamDims D = team_dims(a.la, a.lb, a.lc, a.ld);
-  const int CA = a.team_ca, RPP = a.team_rpp;  // first-shell components per pass, roots per table pass
-  const int nbcd = D.ncb * D.ncc * D.ncd;
-  double *s_x = lds;
-  double *s_w = lds + 16;
-  double *s_H = lds + 32;
-  double *s_I = s_H + RPP * 3 * D.nh;
-  // quartet count: the list's device counter for a launch sized to the
-  // list's capacity before the list was built
-  const long long nq = a.nq_dev ? min((long long)*a.nq_dev - a.nq_base, a.nq) : a.nq;
-  for (long long q = blockIdx.x; q < nq; q += gridDim.x) {
-    const Quartet qt = a.quartets[q];
-    const PairRec bp = a.bra[qt.bra];
-    const PairRec kp = a.ket[qt.ket_mask & 0xFFFFFFu];
-    for (int ia0 = 0; ia0 < D.nca; ia0 += CA) {
-      const int na = D.nca - ia0 < CA ? D.nca - ia0 : CA;
-      const int nsub = na * nbcd;
-      for (int o = lane; o < nsub; o += 64) s_I[o] = 0.0;
-      for (int i = 0; i < bp.npp; ++i) {
-        const PrimPair A = a.prims[bp.pp_off + i];
-        for (int j = 0; j < kp.npp; ++j) {
-          const PrimPair B = a.prims[kp.pp_off + j];
-          const double pq = A.p + B.p, rho = A.p * B.p / pq;
-          const double PQ[3] = {A.P[0] - B.P[0], A.P[1] - B.P[1], A.P[2] - B.P[2]};
-          const double T = rho * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]);
-          const double pref = A.K * B.K * kTwoPi52 / (A.p * B.p * sqrt(pq));
-          __syncthreads();
-          if (lane < D.nr) {
-            double x, w;
-            rys_root_rt(D.nr, lane, T, a.rys, x, w);
-            s_x[lane] = x;
-            s_w[lane] = w * pref;
-          }
-          for (int r0 = 0; r0 < D.nr; r0 += RPP) {
-            const int nrp = D.nr - r0 < RPP ? D.nr - r0 : RPP;
-            __syncthreads();
-            if (lane < 3 * nrp) {
-              const int lr = lane / 3, dir = lane % 3, r = r0 + lr;
-              rys_2d(D, s_x[r], A.p, B.p, A.P[dir] - bp.A[dir], B.P[dir] - kp.A[dir], PQ[dir], bp.AB[dir], kp.AB[dir],
-                     dir == 2 ? s_w[r] : 1.0, s_H + (lr * 3 + dir) * D.nh);
-            }
-            __syncthreads();
-            for (int o = lane; o < nsub; o += 64) {
-              int rem = o;
-              const int id = rem % D.ncd; rem /= D.ncd;
-              const int ic = rem % D.ncc; rem /= D.ncc;
-              const int ib = rem % D.ncb; rem /= D.ncb;
-              const int ia = ia0 + rem;
-              int e[4][3];
-              cart_exp(D.la, ia, e[0][0], e[0][1], e[0][2]);
-              cart_exp(D.lb, ib, e[1][0], e[1][1], e[1][2]);
-              cart_exp(D.lc, ic, e[2][0], e[2][1], e[2][2]);
-              cart_exp(D.ld, id, e[3][0], e[3][1], e[3][2]);
-              int h[3];
-              for (int dir = 0; dir < 3; ++dir)
-                h[dir] = ((e[0][dir] * (D.lb + 1) + e[1][dir]) * (D.lc + 1) + e[2][dir]) * (D.ld + 1) +
-                         e[3][dir];
-              double sum = 0.0;
-              for (int lr = 0; lr < nrp; ++lr) {
-                const double *Hr = s_H + lr * 3 * D.nh;
-                sum += Hr[h[0]] * Hr[D.nh + h[1]] * Hr[2 * D.nh + h[2]];
-              }
-              s_I[o] += sum;
-            }
-          }
-        }
-      }
-      __syncthreads();
-      if (a.store_mode) {
-        double *out = a.store + a.store_off[q] + (size_t)ia0 * nbcd;
-        for (int o = lane; o < nsub; o += 64) out[o] = s_I[o];
-      } else {
-        // degeneracy of the quartet in the 8-fold loop (direct.hpp:1664-1667,
-        // 1793-1802), times the 1/2 of direct.hpp:1849-1850
-        const bool same_pair = (bp.a == kp.a && bp.b == kp.b);
-        const double deg = (bp.a == bp.b ? 1.0 : 2.0) * (kp.a == kp.b ? 1.0 : 2.0) * (same_pair ? 1.0 : 2.0);
-        for (int o = lane; o < nsub; o += 64) s_I[o] *= 0.5 * deg;
-        __syncthreads();
-        // the pass is the quartet of a's components ia0 .. ia0 + na - 1
-        const int n[4] = {na, D.ncb, D.ncc, D.ncd};
-        const int bf[4] = {bp.bfa + ia0, bp.bfb, kp.bfa, kp.bfb};
-        digest_wave(s_I, n, bf, a.planes, qt.ket_mask >> 24, bp.mol, lane, 64);
-      }
-      __syncthreads();
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Screening: quartet candidates (bra i, ket j) after the Schwarz pre-cut,
@@ -622,44 +437,6 @@ __global__ void zero_kernel(double *p, size_t n) {
 inline unsigned nblocks(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 }  // namespace
-
-bool team_shape(int la, int lb, int lc, int ld, int lds_max_bytes, int &ca, int &rpp) {
-  const int nr = (la + lb + lc + ld) / 2 + 1;
-  const int nh = (la + 1) * (lb + 1) * (lc + 1) * (ld + 1);
-  auto nc = [](int l) { return (l + 1) * (l + 2) / 2; };
-  const int nca = nc(la), nbcd = nc(lb) * nc(lc) * nc(ld);
-  const int budget = lds_max_bytes / (int)sizeof(double);
-  // the most first-shell components per pass (fewest passes over the
-  // primitives), then the most roots per table pass that still fit
-  for (ca = nca; ca >= 1; --ca) {
-    if (team_lds_doubles(1, nh, ca, nbcd) > budget) continue;
-    rpp = nr;
-    while (rpp > 1 && team_lds_doubles(rpp, nh, ca, nbcd) > budget) --rpp;
-    return true;
-  }
-  return false;
-}
-
-hipError_t launch_eri_team(const EriLaunch &a0, hipStream_t s) {
-  if (a0.nq <= 0) return hipSuccess;
-  if (a0.la > kMaxLDev || a0.lb > kMaxLDev || a0.lc > kMaxLDev || a0.ld > kMaxLDev) return hipErrorInvalidValue;
-  EriLaunch a = a0;
-  if (!team_shape(a.la, a.lb, a.lc, a.ld, 160 * 1024, a.team_ca, a.team_rpp)) return hipErrorInvalidValue;
-  const int nh = (a.la + 1) * (a.lb + 1) * (a.lc + 1) * (a.ld + 1);
-  auto nc = [](int l) { return (l + 1) * (l + 2) / 2; };
-  const size_t lds = sizeof(double) * (size_t)team_lds_doubles(a.team_rpp, nh, a.team_ca, nc(a.lb) * nc(a.lc) * nc(a.ld));
-  // once per process (contexts on several host threads launch concurrently)
-  static std::once_flag attr_once;
-  static hipError_t attr_err = hipSuccess;
-  std::call_once(attr_once, [] {
-    attr_err = hipFuncSetAttribute((const void *)eri_team_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   160 * 1024);
-  });
-  if (attr_err != hipSuccess) return attr_err;
-  const long long grid = a.nq < 65536 ? a.nq : 65536;
-  hipLaunchKernelGGL(eri_team_kernel, dim3((unsigned)grid), dim3(64), lds, s, a);
-  return hipGetLastError();
-}
 
 hipError_t launch_tile_lists(const TileListLaunch *lists, const long long *start, int nlist, long long nsub,
                              hipStream_t s) {

@@ -24,14 +24,14 @@ constexpr long long kMaxWorkItems = 1ll << 32;
 // Blocks of the generic (team) kernel, which loops over its quartets.
 constexpr long long kTeamGridMax = 65536;
 
-// Threads per block and quartets per block of a family; shape = lanes per
+// Threads per block (at most) and quartets per block of a family; shape = lanes per
 // quartet (lane-group kernels: 1, 2, 4, 8, 16) or quartets per wave (wave
 // kernels: 1, 2, 4, 8).
-inline int family_threads(int family) { return family == kFamilyTeam ? 64 : 256; }
+inline int family_threads(int) { return 256; }
 inline long long quartets_per_block(int family, int shape) {
   if (family == kFamilyLaneGroup) return 4ll * (64 / (shape > 0 ? shape : 1));
   if (family == kFamilyWave) return 4ll * (shape > 0 ? shape : 1);
-  return 1;  // team kernel: one wave per quartet, grid-stride
+  return 1;  // team kernel: one block per quartet, grid-stride
 }
 
 // A lane-group block takes a run of consecutive batches (a batch: the
