@@ -27,8 +27,21 @@ FLAGS = [
 ]
 
 
+def rys_powers(tab):
+    """The Rys table (Chebyshev series in u = 2 (T - i) - 1, rows of NCOEF) in
+    powers of t = T - (i + 1/2) = u / 2, converted in extended precision."""
+    n = 14  # CQX_RYS_NCOEF
+    cheb = np.zeros((n, n), dtype=np.longdouble)  # powers of u of each Chebyshev polynomial
+    cheb[0, 0] = cheb[1, 1] = 1
+    for k in range(2, n):
+        cheb[k, 1:] = 2 * cheb[k - 1, :-1]
+        cheb[k] -= cheb[k - 2]
+    scale = np.longdouble(2) ** np.arange(n)
+    return (tab.reshape(-1, n).astype(np.longdouble) @ cheb * scale).astype(np.float64).ravel()
+
+
 def write_rys_inc():
-    tab = np.fromfile(os.path.join(CSRC, "rys_table.bin"), dtype="<f8")
+    tab = rys_powers(np.fromfile(os.path.join(CSRC, "rys_table.bin"), dtype="<f8"))
     path = os.path.join(CSRC, "rys_table_data.inc")
     with open(path, "w") as f:
         for i in range(0, tab.size, 4):

@@ -148,16 +148,6 @@ template <class R> __device__ __forceinline__ const R *rys_table(const double *r
 template <> __device__ __forceinline__ const double *rys_table<double>(const double *r64, const float *) { return r64; }
 template <> __device__ __forceinline__ const float *rys_table<float>(const double *, const float *r32) { return r32; }
 
-// 1 / sqrt(x): in FP64 the hardware estimate refined by one third-order
-// step (error about one ulp), in FP32 the hardware form.
-template <class R> __device__ __forceinline__ R eval_rsqrt(R x);
-template <> __device__ __forceinline__ double eval_rsqrt<double>(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x, y * y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-template <> __device__ __forceinline__ float eval_rsqrt<float>(float x) { return __builtin_amdgcn_rsqf(x); }
-
 }  // namespace
 
 }  // namespace cqx

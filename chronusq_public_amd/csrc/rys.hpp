@@ -3,8 +3,12 @@
 // For n roots: nodes x_r = t_r^2 in (0, 1) and weights w_r with
 // sum_r w_r x_r^k = F_k(T) for k < 2n (F_k: Boys function).  Below the
 // per-n cut-off T_n the values come from Chebyshev fits on unit intervals
-// of T (table generated by gen_rys_table.py); above it from the
-// Gauss-Hermite asymptotic form x = r^2 / T, w = W / sqrt(T).
+// of T (gen_rys_table.py), which the build rewrites in powers of
+// t = T - (i + 1/2): 13 fused multiply-adds a value, where the Chebyshev
+// recurrence takes 27 operations.  On |t| <= 1/2 the powers fall faster
+// than their rounding matters (the k-th coefficient is the k-th derivative
+// over k!).  Above the cut-off: the Gauss-Hermite asymptotic form
+// x = r^2 / T, w = W / sqrt(T), from one reciprocal square root.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -23,17 +27,24 @@ template <class R> __device__ __forceinline__ R eval_sqrt(R x);
 template <> __device__ __forceinline__ double eval_sqrt<double>(double x) { return sqrt(x); }
 template <> __device__ __forceinline__ float eval_sqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
 
-// R = double, or float for the reduced-precision quartets (table in FP32)
+// 1 / sqrt(x): in FP64 the hardware estimate refined by one third-order
+// step (error about one ulp), in FP32 the hardware form.
+template <class R> __device__ __forceinline__ R eval_rsqrt(R x);
+template <> __device__ __forceinline__ double eval_rsqrt<double>(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x, y * y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+template <> __device__ __forceinline__ float eval_rsqrt<float>(float x) { return __builtin_amdgcn_rsqf(x); }
+
+// A table entry at t = T - (i + 1/2); R = double, or float for the
+// reduced-precision quartets (table in FP32)
 template <class R>
-__device__ __forceinline__ R chebyshev(const R *__restrict__ c, R u) {
-  R b1 = 0, b2 = 0;
+__device__ __forceinline__ R rys_poly(const R *__restrict__ c, R t) {
+  R v = c[CQX_RYS_NCOEF - 1];
 #pragma unroll
-  for (int k = CQX_RYS_NCOEF - 1; k >= 1; --k) {
-    R b0 = fma((R)2 * u, b1, c[k] - b2);
-    b2 = b1;
-    b1 = b0;
-  }
-  return fma(u, b1, c[0] - b2);
+  for (int k = CQX_RYS_NCOEF - 2; k >= 0; --k) v = fma(t, v, c[k]);
+  return v;
 }
 
 // The n-root section of the table: its offset and length (entries)
@@ -51,7 +62,7 @@ __device__ __forceinline__ void rys_roots_sec(R T, const R *__restrict__ tabn, R
                                               R *__restrict__ w) {
   constexpr int kTcut = 34 + 6 * N;
   if (T >= (R)kTcut) {
-    const R rt = eval_rcp<R>(T), rs = eval_sqrt<R>(rt);
+    const R rs = eval_rsqrt<R>(T), rt = rs * rs;
 #pragma unroll
     for (int r = 0; r < N; ++r) {
       x[r] = (R)cqx_rys_asym_x[N][r] * rt;
@@ -59,12 +70,12 @@ __device__ __forceinline__ void rys_roots_sec(R T, const R *__restrict__ tabn, R
     }
   } else {
     const int i = (int)T;
-    const R u = (R)2 * (T - (R)i) - (R)1;
+    const R t = T - ((R)i + (R)0.5);
     const R *c = tabn + (size_t)i * (2 * N * CQX_RYS_NCOEF);
 #pragma unroll
     for (int r = 0; r < N; ++r) {
-      x[r] = chebyshev<R>(c + r * CQX_RYS_NCOEF, u);
-      w[r] = chebyshev<R>(c + (N + r) * CQX_RYS_NCOEF, u);
+      x[r] = rys_poly<R>(c + r * CQX_RYS_NCOEF, t);
+      w[r] = rys_poly<R>(c + (N + r) * CQX_RYS_NCOEF, t);
     }
   }
 }
@@ -75,7 +86,7 @@ __device__ __forceinline__ void rys_roots(R T, const R *__restrict__ tab, R *__r
                                           R *__restrict__ w) {
   constexpr int kTcut = 34 + 6 * N, kOff = rys_tab_off(N);
   if (T >= (R)kTcut) {
-    const R rt = eval_rcp<R>(T), rs = eval_sqrt<R>(rt);
+    const R rs = eval_rsqrt<R>(T), rt = rs * rs;
 #pragma unroll
     for (int r = 0; r < N; ++r) {
       x[r] = (R)cqx_rys_asym_x[N][r] * rt;
@@ -83,12 +94,12 @@ __device__ __forceinline__ void rys_roots(R T, const R *__restrict__ tab, R *__r
     }
   } else {
     const int i = (int)T;
-    const R u = (R)2 * (T - (R)i) - (R)1;
+    const R t = T - ((R)i + (R)0.5);
     const R *c = tab + kOff + (size_t)i * (2 * N * CQX_RYS_NCOEF);
 #pragma unroll
     for (int r = 0; r < N; ++r) {
-      x[r] = chebyshev<R>(c + r * CQX_RYS_NCOEF, u);
-      w[r] = chebyshev<R>(c + (N + r) * CQX_RYS_NCOEF, u);
+      x[r] = rys_poly<R>(c + r * CQX_RYS_NCOEF, t);
+      w[r] = rys_poly<R>(c + (N + r) * CQX_RYS_NCOEF, t);
     }
   }
 }
@@ -99,15 +110,15 @@ template <int N, class R>
 __device__ __forceinline__ void rys_root_sec(R T, const R *__restrict__ tabn, int r, R &x, R &w) {
   constexpr int kTcut = 34 + 6 * N;
   if (T >= (R)kTcut) {
-    const R rt = eval_rcp<R>(T);
-    x = (R)cqx_rys_asym_x[N][r] * rt;
-    w = (R)cqx_rys_asym_w[N][r] * eval_sqrt<R>(rt);
+    const R rs = eval_rsqrt<R>(T);
+    x = (R)cqx_rys_asym_x[N][r] * (rs * rs);
+    w = (R)cqx_rys_asym_w[N][r] * rs;
   } else {
     const int i = (int)T;
-    const R u = (R)2 * (T - (R)i) - (R)1;
+    const R t = T - ((R)i + (R)0.5);
     const R *c = tabn + (size_t)i * (2 * N * CQX_RYS_NCOEF);
-    x = chebyshev<R>(c + r * CQX_RYS_NCOEF, u);
-    w = chebyshev<R>(c + (N + r) * CQX_RYS_NCOEF, u);
+    x = rys_poly<R>(c + r * CQX_RYS_NCOEF, t);
+    w = rys_poly<R>(c + (N + r) * CQX_RYS_NCOEF, t);
   }
 }
 // the same from the whole table
@@ -123,17 +134,17 @@ __device__ __forceinline__ void rys_root_rt(int n, int r, double T,
                                             double &x, double &w) {
   const int tcut = 34 + 6 * n;  // 40, 46, ..., 88
   if (T >= (double)tcut) {
-    const double rt = 1.0 / T;
-    x = cqx_rys_asym_x_dev(n, r) * rt;
-    w = cqx_rys_asym_w_dev(n, r) * sqrt(rt);
+    const double rs = eval_rsqrt<double>(T);
+    x = cqx_rys_asym_x_dev(n, r) * (rs * rs);
+    w = cqx_rys_asym_w_dev(n, r) * rs;
   } else {
     int off = 0;
     for (int k = 1; k < n; ++k) off += (34 + 6 * k) * 2 * k * CQX_RYS_NCOEF;
     const int i = (int)T;
-    const double u = 2.0 * (T - (double)i) - 1.0;
+    const double t = T - ((double)i + 0.5);
     const double *c = tab + off + (size_t)i * (2 * n * CQX_RYS_NCOEF);
-    x = chebyshev<double>(c + r * CQX_RYS_NCOEF, u);
-    w = chebyshev<double>(c + (n + r) * CQX_RYS_NCOEF, u);
+    x = rys_poly<double>(c + r * CQX_RYS_NCOEF, t);
+    w = rys_poly<double>(c + (n + r) * CQX_RYS_NCOEF, t);
   }
 }
 
