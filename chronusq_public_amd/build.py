@@ -51,7 +51,7 @@ def write_rys_inc():
 
 # the sources of the ERI + digestion launches of a Fock build: the kernels,
 # their headers and the Rys table
-KERNEL_SOURCES = ("eri_", "digest", "kernels.", "device_types.hpp", "rys.hpp", "rys_table.bin", "cand.hip",
+KERNEL_SOURCES = ("eri_", "digest", "kernels.", "device_types.hpp", "rys.hpp", "rys_table.bin", "front.",
                   "limits.hpp")
 
 

@@ -22,6 +22,7 @@
 #include "basis.hpp"
 #include "device_types.hpp"
 #include "eri_row.hpp"
+#include "front.hpp"
 #include "kernels.hpp"
 #include "onebody.hpp"
 #include "ctx_access.hpp"
@@ -76,6 +77,21 @@ using cqx::PrimPair;
 using cqx::Quartet;
 
 namespace {
+
+// Host matrices of a build are gathered into one copy each way up to this
+// many bytes of densities (and as many of outputs): four small pageable
+// copies cost 0.06-0.1 ms (water / 6-31G(d) 0.50 -> 0.44 ms, the five complex
+// matrices of (H2O)3 / STO-3G 0.42 -> 0.33); with larger matrices the extra
+// pass over host memory and the saved copies come out even ((H2O)4 / cc-pVDZ
+// 0.79 both ways)
+constexpr size_t kGatherBytes = 1 << 20;
+// Quartet-list class pairs are launched over their list's capacity, without
+// reading candidate totals and list counts back in between, when all pairs
+// of pairs are at most this many (8 MB of list): the two waits saved are
+// worth 0.07 ms (water / 6-31G(d) 0.50 -> 0.44, (H2O)4 / cc-pVDZ 0.82 ->
+// 0.79), the empty wavefronts of larger lists cost more ((H2O)6 / cc-pVTZ
+// 10.27 -> 10.42 ms with 16 M)
+constexpr long long kSmallLists = 1 << 20;
 
 // LDS of a row block beyond which a class pair takes quartet lists: all a
 // block can have (one block per CU still beats the lists: GHF (ps|ps) of
@@ -184,11 +200,18 @@ struct cqx_ctx {
   cqx::CartMap cmap{};
 
   // per-call workspace
-  DevBuf<double> d_X, d_AX, d_Bm, d_Bg, d_planes, d_acc;
-  DevBuf<int> d_her;
+  DevBuf<double> d_X, d_Bm, d_Bg, d_planes, d_acc;
   DevBuf<long long> d_cand, d_mol_boff;
   DevBuf<int> d_mol_ns, d_ket_lo, d_seg;
-  DevBuf<char> d_scan_tmp;
+  DevBuf<cqx::CandLaunch> d_cands;
+  DevBuf<const double *> d_px;
+  DevBuf<double *> d_pa;
+  DevBuf<double> d_small;
+  // what the tables above (and the plane table) last held, so that a build
+  // with the same ones uploads nothing
+  std::vector<char> kept_cands, kept_px, kept_pa, kept_molplanes, kept_lists, kept_lstart;
+  std::vector<cqx::MolInfo> molinfo;  // nmol + 1: the last entry holds the totals
+  DevBuf<cqx::MolInfo> d_molinfo;
   DevBuf<cqx::ListLaunch> d_lists;
   DevBuf<long long> d_lstart;
   DevBuf<double> d_molmax;
@@ -200,16 +223,16 @@ struct cqx_ctx {
   DevBuf<long long> d_store_off;
   DevBuf<double> d_jx, d_ja;                  // row kernels: Coulomb planes in pair order
   DevBuf<double> d_rcount;                    // per row launch: quartets, candidates (integers), primitive sum
-  DevBuf<long long> d_tidx, d_tot;  // candidate totals of an eager build, gathered for one copy
+  DevBuf<long long> d_tot;  // candidate totals
   // The workspace of the contraction group in flight: views of the buffers
   // above (allocated on demand) or of a fixed scratch region
   struct Ws {
     double *X, *AX, *Bm, *Bg, *molmax, *planes, *acc;
     double *pn[kNumClass];
-    int *her, *ket_lo;
-    long long *cand, *tidx, *tot, *lstart;
-    void *scan;
-    size_t scan_bytes;
+    int *ket_lo;
+    long long *cand, *tot, *lstart;
+    cqx::CandLaunch *cands;
+    double *small;
     cqx::MolPlanes *molplanes;
     Quartet *quart;
     unsigned long long *count;
@@ -241,13 +264,14 @@ struct cqx_ctx {
   std::string graph_key;           // contraction signature of the recording build
   int g_nmat = 0, g_nJ = 0, g_nK = 0;
   bool g_pure_d = false;
+  size_t g_x = 0;                      // doubles of the staged densities (the staged outputs follow them)
   std::vector<size_t> g_xoff, g_mnb2;  // per molecule: offset and size of its matrices
   std::vector<long long> g_cap;        // per class pair: candidate capacity
   std::vector<long long> g_lcap;       // per ERI slot: list capacity
   std::vector<GraphSlot> g_rows;       // per row launch
   std::vector<GraphSlot> g_slots;      // per ERI slot (class pair, precision); la < 0: not launched
   DevBuf<cqx::ListLaunch> d_glists;
-  DevBuf<long long> d_glstart, d_gidx, d_gchk;
+  DevBuf<long long> d_glstart;
 
   // Tiles (option "tiles", default 0): the lane-group class pairs of a
   // build whose planes are all Hermitian go through tile lists instead of
@@ -506,6 +530,24 @@ void setup_device_maps(cqx_ctx *c) {
     mns[m] = B.mol_sh0[m + 1] - B.mol_sh0[m];
     c->mol_boff[m + 1] = c->mol_boff[m] + (long long)mns[m] * mns[m];
   }
+  c->molinfo.assign(c->nmol + 1, cqx::MolInfo{});
+  for (int m = 0; m <= c->nmol; ++m) {
+    cqx::MolInfo &I = c->molinfo[m];
+    I.boff = c->mol_boff[m];
+    if (m > 0) {
+      const cqx::MolInfo &P = c->molinfo[m - 1];
+      I.nb2 = P.nb2 + (long long)P.nb * P.nb;
+      I.nbc2 = P.nbc2 + (long long)P.nbc * P.nbc;
+    }
+    if (m == c->nmol) break;
+    I.nb = B.mol_bf0[m + 1] - B.mol_bf0[m];
+    I.nbc = B.mol_bfc0[m + 1] - B.mol_bfc0[m];
+    I.ns = mns[m];
+    I.bf0 = B.mol_bf0[m];
+    I.bfc0 = B.mol_bfc0[m];
+    I.sh0 = B.mol_sh0[m];
+  }
+  c->d_molinfo.upload(c->molinfo, c->stream);
   c->d_mol_ns.upload(mns, c->stream);
   c->d_mol_boff.upload(c->mol_boff, c->stream);
 }
@@ -810,7 +852,7 @@ bool replay_graph(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_comp
       const cqx_contraction &cc = list[m * nper + j];
       const size_t o = c->g_xoff[m] + (size_t)j * c->g_mnb2[m] * ew, n = sizeof(double) * c->g_mnb2[m] * ew;
       HIPCHK(hipMemcpyAsync(c->d_X.p + o, cc.X, n, hk, s));
-      HIPCHK(hipMemcpyAsync(c->d_AX.p + o, cc.AX, n, hk, s));
+      HIPCHK(hipMemcpyAsync(c->d_X.p + c->g_x + o, cc.AX, n, hk, s));
     }
   HIPCHK(hipEventRecord(c->ev0, s));
   HIPCHK(hipGraphLaunch(c->graph_exec, s));
@@ -820,7 +862,7 @@ bool replay_graph(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_comp
   std::vector<unsigned long long> counts(2 * ncp), rcount(3 * c->g_rows.size());
   std::vector<double> psum(2 * ncp);
   if (ncp) {
-    HIPCHK(hipMemcpyAsync(tot.data(), c->d_gchk.p, sizeof(long long) * ncp, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(tot.data(), c->d_tot.p, sizeof(long long) * ncp, hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(counts.data(), c->d_count.p, sizeof(unsigned long long) * 2 * ncp, hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(psum.data(), c->d_psum.p, sizeof(double) * 2 * ncp, hipMemcpyDeviceToHost, s));
   }
@@ -834,7 +876,7 @@ bool replay_graph(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_comp
   const hipMemcpyKind dk = mem == CQX_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
   for (int m = 0; m < nmol; ++m)
     for (int j = 0; j < nmat; ++j)
-      HIPCHK(hipMemcpyAsync(list[m * nper + j].AX, c->d_AX.p + c->g_xoff[m] + (size_t)j * c->g_mnb2[m] * ew,
+      HIPCHK(hipMemcpyAsync(list[m * nper + j].AX, c->d_X.p + c->g_x + c->g_xoff[m] + (size_t)j * c->g_mnb2[m] * ew,
                             sizeof(double) * c->g_mnb2[m] * ew, dk, s));
   HIPCHK(hipStreamSynchronize(s));
   float ms = 0.0f;
@@ -1296,14 +1338,13 @@ struct GroupPlan {
   size_t planes = 0;  // doubles of the Cartesian planes (and of the accumulators)
   size_t cand = 0;    // candidate offsets (long long) and first kets (int)
   size_t ncp = 0;     // class pairs with pairs on both sides
-  size_t scan_bytes = 0;
   long long max_ket = 0;   // largest ket class of a class pair
   long long cand_all = 0;  // candidates of every class pair without the Schwarz pre-cut
   int kcnt[4] = {0, 0, 0, 0};
   int kps[4] = {1, 1, 1, 1};
 };
 
-GroupPlan plan_group(const cqx_ctx *c, const cqx_contraction *L, int nmat, int is_complex, hipStream_t s) {
+GroupPlan plan_group(const cqx_ctx *c, const cqx_contraction *L, int nmat, int is_complex) {
   GroupPlan g;
   g.nmat = nmat;
   const cqx::Basis &BS = c->basis;
@@ -1338,11 +1379,6 @@ GroupPlan plan_group(const cqx_ctx *c, const cqx_contraction *L, int nmat, int i
       ++g.ncp;
       g.max_ket = std::max(g.max_ket, nket);
       g.cand_all += nbra * nket;
-      cqx::CandLaunch CL{};
-      CL.nbra = (int)nbra;
-      size_t b = 0;
-      HIPCHK(cqx::launch_candidates(CL, nullptr, b, s));  // size query only
-      g.scan_bytes = std::max(g.scan_bytes, b);
     }
   return g;
 }
@@ -1359,15 +1395,25 @@ long long list_entries_bound(const GroupPlan &g, long long list_cap) {
 size_t workspace_bytes(const cqx_ctx *c) {
   size_t b = 0;
   auto add = [&](const auto &buf) { b += buf.n * sizeof(*buf.p); };
-  add(c->d_X); add(c->d_AX); add(c->d_Bm); add(c->d_Bg); add(c->d_planes); add(c->d_acc);
-  add(c->d_her); add(c->d_cand); add(c->d_ket_lo); add(c->d_scan_tmp); add(c->d_lists);
+  add(c->d_X); add(c->d_Bm); add(c->d_Bg); add(c->d_planes); add(c->d_acc);
+  add(c->d_cand); add(c->d_ket_lo); add(c->d_cands); add(c->d_px); add(c->d_pa); add(c->d_small); add(c->d_lists);
   add(c->d_lstart); add(c->d_molmax); add(c->d_molplanes); add(c->d_quart); add(c->d_count);
-  add(c->d_psum); add(c->d_tidx); add(c->d_tot); add(c->d_acc_tune); add(c->d_molplanes_tune);
-  add(c->d_glists); add(c->d_glstart); add(c->d_gidx); add(c->d_gchk);
+  add(c->d_psum); add(c->d_tot); add(c->d_acc_tune); add(c->d_molplanes_tune);
+  add(c->d_glists); add(c->d_glstart);
   add(c->d_jx); add(c->d_ja); add(c->d_rcount);
   add(c->d_tiles); add(c->d_tcount); add(c->d_tpsum); add(c->d_tll); add(c->d_tstart);
   for (int k = 0; k < kNumClass; ++k) add(c->d_pn[k]);
   return b;
+}
+
+// Whether kernels on the device can take p: memory of that device.
+bool on_device(const void *p, int device) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == device;
 }
 
 // Upload a host array into a workspace view (the context's buffer, grown
@@ -1383,6 +1429,22 @@ T *ws_upload(DevBuf<T> &buf, Arena *scr, const std::vector<T> &v, hipStream_t s,
   }
   if (!v.empty()) HIPCHK(hipMemcpyAsync(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, s));
   return p;
+}
+// The same for a table that rarely changes between builds of a context: kept
+// holds the bytes the context's buffer last received.
+template <class T>
+T *ws_upload_kept(DevBuf<T> &buf, std::vector<char> &kept, Arena *scr, const std::vector<T> &v, hipStream_t s,
+                  const char *what) {
+  if (scr) return ws_upload(buf, scr, v, s, what);
+  const size_t n = sizeof(T) * v.size();
+  if (buf.p && buf.n >= v.size() && kept.size() == n && (n == 0 || std::memcmp(kept.data(), v.data(), n) == 0))
+    return buf.p;
+  kept.clear();
+  buf.ensure(std::max<size_t>(v.size(), 1));
+  std::vector<char> bytes(reinterpret_cast<const char *>(v.data()), reinterpret_cast<const char *>(v.data()) + n);
+  if (n) HIPCHK(hipMemcpyAsync(buf.p, bytes.data(), n, hipMemcpyHostToDevice, s));
+  kept.swap(bytes);  // the copy's source stays in place
+  return buf.p;
 }
 template <class T>
 T *ws_take(DevBuf<T> &buf, Arena *scr, size_t n, const char *what) {
@@ -1453,28 +1515,55 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       int nplane = 0;
       const int nmat = group_size(list + start, nper - start, is_complex, &nplane);
       const cqx_contraction *L = list + start;  // molecule 0's contractions of the group
-      const GroupPlan gp = plan_group(c, L, nmat, is_complex, s);
+      const GroupPlan gp = plan_group(c, L, nmat, is_complex);
       if (scr) scr->used = 0;  // each group reuses the whole region
       // densities (and, when allocating, the outputs) on the device:
       // molecule m's nmat matrices at xoff[m]
       std::vector<size_t> xoff(nmol + 1, 0);
       for (int m = 0; m < nmol; ++m) xoff[m + 1] = xoff[m] + (size_t)nmat * mnb2[m] * ew;
-      w.X = ws_take(c->d_X, scr, gp.x, "the staged densities");
-      w.AX = scr ? nullptr : ws_take(c->d_AX, scr, gp.x, "the staged outputs");
-      const hipMemcpyKind hk = mem == CQX_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+      // Device matrices are read and added to in place (read through a copy
+      // in the allocation-free build), unless the build is recorded (a replay
+      // works on the staged copies), memory is not this device's own, or two
+      // contractions share an output (each then adds to its own copy, and the
+      // last one stays).
+      std::vector<std::pair<const char *, size_t>> outs;
       for (int m = 0; m < nmol; ++m)
-        for (int j = 0; j < nmat; ++j) {
-          const cqx_contraction &cc = list[m * nper + start + j];
-          const size_t o = xoff[m] + (size_t)j * mnb2[m] * ew, n = sizeof(double) * mnb2[m] * ew;
-          HIPCHK(hipMemcpyAsync(w.X + o, cc.X, n, hk, s));
-          if (!scr) HIPCHK(hipMemcpyAsync(w.AX + o, cc.AX, n, hk, s));
-        }
+        for (int j = 0; j < nmat; ++j)
+          outs.push_back({static_cast<const char *>(list[m * nper + start + j].AX), sizeof(double) * mnb2[m] * ew});
+      std::sort(outs.begin(), outs.end());
+      bool shared = false;
+      for (size_t k = 1; k < outs.size(); ++k) shared = shared || outs[k - 1].first + outs[k - 1].second > outs[k].first;
+      bool direct = !scr && mem == CQX_DEVICE && !c->use_graph && !shared;
+      for (int i = 0; direct && i < nmol * nmat; ++i) {
+        const cqx_contraction &cc = list[(i / nmat) * nper + start + i % nmat];
+        direct = on_device(cc.X, c->device) && on_device(cc.AX, c->device);
+      }
+      const bool in_place = direct || scr;  // the outputs
+      w.X = w.AX = nullptr;
+      // host matrices of a small build go through one gathered copy each way
+      const bool gather = !in_place && mem == CQX_HOST && sizeof(double) * gp.x <= kGatherBytes;
+      std::vector<double> hbuf;
+      if (!direct) {
+        w.X = ws_take(c->d_X, scr, scr ? gp.x : 2 * gp.x, "the staged densities and outputs");
+        w.AX = scr ? nullptr : w.X + gp.x;
+        if (gather) hbuf.resize(2 * gp.x);
+        const hipMemcpyKind hk = mem == CQX_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+        for (int m = 0; m < nmol; ++m)
+          for (int j = 0; j < nmat; ++j) {
+            const cqx_contraction &cc = list[m * nper + start + j];
+            const size_t o = xoff[m] + (size_t)j * mnb2[m] * ew, n = sizeof(double) * mnb2[m] * ew;
+            if (gather) {
+              std::memcpy(hbuf.data() + o, cc.X, n);
+              std::memcpy(hbuf.data() + gp.x + o, cc.AX, n);
+            } else {
+              HIPCHK(hipMemcpyAsync(w.X + o, cc.X, n, hk, s));
+              if (!scr) HIPCHK(hipMemcpyAsync(w.AX + o, cc.AX, n, hk, s));
+            }
+          }
+        if (gather) HIPCHK(hipMemcpyAsync(w.X, hbuf.data(), sizeof(double) * hbuf.size(), hipMemcpyHostToDevice, s));
+      }
       // --- plan: every upload and allocation of the build comes first, so
       // that the launches below can also be recorded into a graph ---
-      std::vector<int> her(nmat);
-      for (int j = 0; j < nmat; ++j) her[j] = L[j].her ? 1 : 0;
-      w.her = ws_upload(c->d_her, scr, her, s, "the HER flags");
-      const long long nbl = c->mol_boff[nmol];
       w.Bm = ws_take(c->d_Bm, scr, gp.bm, "the shell-block norms");
       w.Bg = ws_take(c->d_Bg, scr, gp.bg, "the shell-block norms");
       w.molmax = ws_take(c->d_molmax, scr, (size_t)nmol, "the molecule norms");
@@ -1526,7 +1615,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         }
         mp[m].nbc = mnbc[m];
       }
-      w.molplanes = ws_upload(c->d_molplanes, scr, mp, s, "the molecule plane table");
+      w.molplanes = ws_upload_kept(c->d_molplanes, c->kept_molplanes, scr, mp, s, "the molecule plane table");
       ps.mols = w.molplanes;
       ps.m0 = mp[0];
       ps.nmol = nmol;
@@ -1545,21 +1634,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         if (P.sign < 0.0) ps.negs |= 1u << p;
       }
       ps.n = nplane;
-      // Cartesian planes of every molecule (real and imaginary planes of a
-      // contraction share a kind, hence a stride)
-      auto mol_map = [&](int m) {
-        cqx::CartMap M = c->cmap;
-        M.cart_shell += BS.mol_bfc0[m];
-        M.cart_comp += BS.mol_bfc0[m];
-        M.bf_shell += BS.mol_bf0[m];
-        M.bf_comp += BS.mol_bf0[m];
-        M.nb = mnb[m];
-        M.nbc = mnbc[m];
-        M.ns = mns[m];
-        M.bf0 = BS.mol_bf0[m];
-        M.bfc0 = BS.mol_bfc0[m];
-        return M;
-      };
       int nJ = 0, nK = 0;
       for (int j = 0; j < nmat; ++j) (L[j].type == CQX_COULOMB ? nJ : nK)++;
       // candidate lists per class pair (bra class >= ket class): bra i of
@@ -1642,8 +1716,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         }
       w.cand = ws_take(c->d_cand, scr, cand_total, "the candidate offsets");
       w.ket_lo = ws_take(c->d_ket_lo, scr, cand_total, "the candidate offsets");
-      w.scan = ws_take(c->d_scan_tmp, scr, gp.scan_bytes, "the scan workspace");
-      w.scan_bytes = std::max<size_t>(gp.scan_bytes, 1);
       std::vector<cqx::CandLaunch> cls_launch(cps.size());
       for (size_t k = 0; k < cps.size(); ++k) {
         const auto &cp = cps[k];
@@ -1661,48 +1733,22 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         CL.off = w.cand + cp.coff;
         CL.klo = w.ket_lo + cp.coff;
       }
-      std::vector<long long> tidx(cps.size());
-      for (size_t k = 0; k < cps.size(); ++k) tidx[k] = (long long)(cps[k].coff + cps[k].nbra);
-      if (!cps.empty()) {
-        w.tidx = ws_upload(c->d_tidx, scr, tidx, s, "the candidate totals");
-        w.tot = ws_take(c->d_tot, scr, cps.size(), "the candidate totals");
+      // a small build: lists launched over their capacities
+      long long cap_all = 0;
+      bool wide = true;  // no lane-group class among them (its shape follows the counts)
+      for (const auto &cp : cps) {
+        int la_, lb_, lc_, ld_;
+        class_ls(cp.cb, la_, lb_);
+        class_ls(cp.ck, lc_, ld_);
+        cap_all += (long long)cp.nbra * (long long)c->cls[cp.ck].size();
+        wide = wide && !cqx::eri_lane_group_built(la_, lb_, lc_, ld_);
       }
-      // AX of the outputs: the staged copies, or the caller's own device
-      // matrices for the allocation-free entry point
-      auto ax_of = [&](int m, int j) -> double * {
-        if (scr) return static_cast<double *>(list[m * nper + start + j].AX);
-        return w.AX + xoff[m] + (size_t)j * mnb2[m] * ew;
-      };
-      // --- launches up to the candidate counts: shell-block norms, per
-      // molecule, and each molecule's largest one; the pairs' own norms;
-      // cleared accumulators; Cartesian density planes; candidate offsets ---
-      auto front = [&]() {
-        for (int m = 0; m < nmol; ++m)
-          HIPCHK(cqx::launch_block_norms(w.X + xoff[m], nmat, is_complex, w.her, mnb[m], mns[m],
-                                         c->d_sh_bf.p + BS.mol_sh0[m], BS.mol_bf0[m], c->d_sh_nf.p + BS.mol_sh0[m],
-                                         w.Bm + (size_t)c->mol_boff[m] * nmat, w.Bg + c->mol_boff[m], s));
-        HIPCHK(cqx::launch_mol_max(w.Bg, c->d_mol_boff.p, c->d_mol_ns.p, nmol, w.molmax, s));
-        for (int k = 0; k < kNumClass; ++k)
-          if (!c->cls[k].empty())
-            HIPCHK(cqx::launch_pair_norms(c->d_scr[k].p, (int)c->cls[k].size(), w.Bg, w.Bm, c->d_mol_boff.p,
-                                          c->d_mol_ns.p, nmat, w.pn[k], s));
-        HIPCHK(cqx::launch_zero(w.acc, poff[nmol], s));
-        for (int m = 0; m < nmol; ++m) {
-          const cqx::CartMap M = mol_map(m);
-          for (int j = 0; j < nmat; ++j) {
-            const int pr = slot_re[j], pi = slot_im[j];
-            double *xre = const_cast<double *>(mp[m].kx[pd[pr].kind]) + pidx[pr];
-            double *xim = pi >= 0 ? const_cast<double *>(mp[m].kx[pd[pi].kind]) + pidx[pi] : nullptr;
-            HIPCHK(cqx::launch_to_cart(M, w.X + xoff[m] + (size_t)j * mnb2[m] * ew, is_complex, xre, xim,
-                                       ps.kps[pd[pr].kind], s));
-          }
-        }
-        for (auto &CL : cls_launch) {
-          size_t b = w.scan_bytes;
-          HIPCHK(cqx::launch_candidates(CL, w.scan, b, s));
-        }
-      };
-      front();
+      const bool small = !rcps.empty() && !cps.empty() && tcps.empty() && wide && !scr && !c->use_graph &&
+                         !c->autotune_pending && cap_all <= std::min(c->list_cap, kSmallLists);
+      const size_t nslots = 2 * cps.size();
+      w.small = small ? ws_take(c->d_small, nullptr, 2 * nslots, "the list counters") : nullptr;
+      w.cands = ws_upload_kept(c->d_cands, c->kept_cands, scr, cls_launch, s, "the candidate launch table");
+      w.tot = ws_take(c->d_tot, scr, std::max<size_t>(cps.size(), 1), "the candidate totals");
       const bool mixed = c->fp32_cut > 0.0;
       const int qmul = mixed ? 2 : 1;  // quartet lists per class pair
       auto ensure_side = [&](int nst) { ensure_sides(c, nst); };
@@ -1718,27 +1764,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       size_t joff[kNumClass + 1] = {};
       std::vector<cqx_ctx::GraphSlot> row_slots;
       std::vector<unsigned long long> rcount;  // per launch: quartets, candidates, primitive sum (a double)
-      auto pair_order = [&](int k) {
-        cqx::PairOrder po{};
-        int la_, lb_;
-        class_ls(k, la_, lb_);
-        po.pairs = c->d_pairs[k].p;
-        po.npair = (int)c->cls[k].size();
-        po.na = cqx::ncart(la_);
-        po.nb = cqx::ncart(lb_);
-        po.m0 = mp[0];
-        po.mols = w.molplanes;
-        po.nmol = nmol;
-        for (int p = 0; p < (int)pd.size(); ++p)
-          if (pd[p].kind == cqx::kJHer || pd[p].kind == cqx::kJNonHer) {
-            po.kind[po.nj] = pd[p].kind;
-            po.idx[po.nj] = pidx[p];
-            po.stride[po.nj++] = ps.kps[pd[p].kind];
-          }
-        po.jx = c->d_jx.p + joff[k];
-        po.ja = c->d_ja.p + joff[k];
-        return po;
-      };
       if (nrow) {
         for (int k = 0; k < kNumClass; ++k) {
           int la_, lb_;
@@ -1752,13 +1777,81 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         rcount.resize(3 * nslot);
         ensure_side(nst_all);
       }
-      auto rows_front = [&]() {
-        if (!nrow) return;
-        HIPCHK(cqx::launch_zero(c->d_rcount.p, rcount.size(), s));
-        HIPCHK(cqx::launch_zero(c->d_ja.p, joff[kNumClass], s));
-        for (int k = 0; k < kNumClass; ++k)
-          if (!c->cls[k].empty() && row0.nj) HIPCHK(cqx::launch_pair_pack(pair_order(k), s));
+      // --- launches up to the candidate counts: shell-block norms and each
+      // molecule's largest one; cleared accumulators; Cartesian density
+      // planes; the pairs' own norms and pair-order Coulomb planes; candidate
+      // offsets ---
+      cqx::FrontArgs fa{};
+      fa.mol = c->d_molinfo.p;
+      fa.nmol = nmol;
+      fa.nmat = nmat;
+      fa.cplx = is_complex;
+      fa.map = c->cmap;
+      fa.sh_nf = c->d_sh_nf.p;
+      std::vector<const double *> px;
+      std::vector<double *> pa;
+      for (int m = 0; m < nmol; ++m)
+        for (int j = 0; j < nmat; ++j) {
+          const cqx_contraction &cc = list[m * nper + start + j];
+          const size_t o = xoff[m] + (size_t)j * mnb2[m] * ew;
+          px.push_back(direct ? static_cast<const double *>(cc.X) : w.X + o);
+          pa.push_back(in_place ? static_cast<double *>(cc.AX) : w.AX + o);
+        }
+      if (nmol == 1) {
+        std::copy(px.begin(), px.end(), fa.xs);
+        std::copy(pa.begin(), pa.end(), fa.axs);
+      } else {
+        fa.x = ws_upload_kept(c->d_px, c->kept_px, scr, px, s, "the matrix table");
+        fa.ax = ws_upload_kept(c->d_pa, c->kept_pa, scr, pa, s, "the matrix table");
+      }
+      fa.m0 = mp[0];
+      fa.mols = w.molplanes;
+      for (int k = 0; k < 4; ++k) fa.kps[k] = ps.kps[k];
+      for (int j = 0; j < nmat; ++j) {
+        if (L[j].her) fa.her |= 1u << j;
+        fa.kind[j] = pd[slot_re[j]].kind;
+        fa.re[j] = pidx[slot_re[j]];
+        fa.im[j] = slot_im[j] >= 0 ? pidx[slot_im[j]] : -1;
+      }
+      fa.Bm = w.Bm;
+      fa.Bg = w.Bg;
+      fa.molmax = w.molmax;
+      for (int k = 0; k < kNumClass; ++k) {
+        int la_, lb_;
+        class_ls(k, la_, lb_);
+        fa.scr[k] = c->d_scr[k].p;
+        fa.pairs[k] = c->d_pairs[k].p;
+        fa.pn[k] = w.pn[k];
+        fa.npair[k] = (int)c->cls[k].size();
+        fa.cstart[k + 1] = fa.cstart[k] + (long long)cqx::ncart(la_) * cqx::ncart(lb_) * fa.npair[k];
+        fa.joff[k] = joff[k];
+      }
+      if (nrow)
+        for (int p = 0; p < (int)pd.size(); ++p)
+          if (pd[p].kind == cqx::kJHer || pd[p].kind == cqx::kJNonHer) {
+            fa.jkind[fa.nj] = pd[p].kind;
+            fa.jidx[fa.nj++] = pidx[p];
+          }
+      if (nrow && fa.nj) {
+        fa.jx = c->d_jx.p;
+        fa.ja = c->d_ja.p;
+      }
+      const long long nb2_all = (long long)c->molinfo[nmol].nb2, nbc2_all = (long long)c->molinfo[nmol].nbc2;
+      auto front = [&]() {
+        cqx::ZeroRanges z;
+        z.add(w.acc, poff[nmol]);
+        z.add(w.molmax, nmol);
+        if (nrow) {
+          z.add(c->d_rcount.p, rcount.size());
+          z.add(c->d_ja.p, joff[kNumClass]);
+        }
+        if (small) z.add(w.small, 2 * nslots);
+        HIPCHK(cqx::launch_zero_ranges(z, s));
+        HIPCHK(cqx::launch_norms(fa, c->mol_boff[nmol], s));
+        HIPCHK(cqx::launch_planes(fa, nbc2_all, s));
+        HIPCHK(cqx::launch_pairs(fa, s));
       };
+      front();
       // every row launch; stream(k): the stream of the k-th
       auto rows_launch = [&](const std::function<hipStream_t(int)> &stream) {
         int nl = 0;
@@ -1814,12 +1907,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           }
         return nl;
       };
-      auto rows_back = [&]() {
-        if (nrow && row0.nj)
-          for (int k = 0; k < kNumClass; ++k)
-            if (!c->cls[k].empty()) HIPCHK(cqx::launch_pair_unpack(pair_order(k), s));
-      };
-      rows_front();
       if (nrow) {
         HIPCHK(hipEventRecord(c->ev_r0, s));
         fork_side(nst_all);
@@ -1876,14 +1963,16 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         HIPCHK(hipMemcpyAsync(tcount.data(), tcnt, sizeof(unsigned long long) * tcount.size(), hipMemcpyDeviceToHost, s));
         HIPCHK(hipMemcpyAsync(tpsum.data(), tps, sizeof(double) * tpsum.size(), hipMemcpyDeviceToHost, s));
       }
-      // every class pair's candidate total (the last entry of its offsets),
-      // gathered on the device and read back in one copy
+      // every class pair's candidate total, read back in one copy
       std::vector<long long> totals(cps.size());
       if (!cps.empty()) {
-        HIPCHK(cqx::launch_gather(w.cand, w.tidx, (int)cps.size(), w.tot, s));
-        HIPCHK(hipMemcpyAsync(totals.data(), w.tot, sizeof(long long) * cps.size(), hipMemcpyDeviceToHost, s));
+        HIPCHK(cqx::launch_candidates_all(w.cands, (int)cps.size(), w.tot, s));
+        if (small)
+          for (size_t k = 0; k < cps.size(); ++k) totals[k] = (long long)cps[k].nbra * (long long)c->cls[cps[k].ck].size();
+        else
+          HIPCHK(hipMemcpyAsync(totals.data(), w.tot, sizeof(long long) * cps.size(), hipMemcpyDeviceToHost, s));
       }
-      if (nt || !cps.empty()) HIPCHK(hipStreamSynchronize(s));
+      if (nt || (!cps.empty() && !small)) HIPCHK(hipStreamSynchronize(s));
       // entries of one list batch: the option, or what the scratch region
       // leaves after this group's fixed workspace (less a reserve for the
       // per-batch tables)
@@ -1905,7 +1994,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           HIPCHK(hipStreamSynchronize(s));
         }
       }
-      c->stats.n_candidates += total;
+      if (!small) c->stats.n_candidates += total;
       for (int k = 0; k < nt; ++k) c->stats.n_candidates += (long long)tcount[3 * k + 2];
       // autotuned shapes: key of a class and precision, and the value tag of
       // a wave shape for the classes built in both families
@@ -1992,24 +2081,18 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       auto launch_eri = [&](const cqx::EriLaunch &E, hipStream_t st) {
         launch_family(E, route(E.la, E.lb, E.lc, E.ld, E.fp32), st);
       };
-      // --- back to pure functions, symmetrise, accumulate into AX: the
-      // contractions' transforms are independent and are dealt over nst
-      // streams like the ERI launches (side streams already created) ---
-      auto back = [&](int nst) {
-        fork_side(nst);
-        int q = 0;
-        for (int m = 0; m < nmol; ++m) {
-          const cqx::CartMap M = mol_map(m);
-          for (int j = 0; j < nmat; ++j) {
-            const bool two = is_complex && !(L[j].her && L[j].type == CQX_COULOMB);
-            const int pr = slot_re[j], pi = slot_im[j];
-            const double *are = mp[m].ka[pd[pr].kind] + pidx[pr];
-            const double *aim = two ? mp[m].ka[pd[pi].kind] + pidx[pi] : nullptr;
-            HIPCHK(cqx::launch_from_cart(M, are, aim, ps.kps[pd[pr].kind], L[j].her, is_complex, ax_of(m, j),
-                                         stream_of(q++, nst)));
-          }
+      // --- pair-order Coulomb sums onto the accumulators, back to pure
+      // functions, symmetrise, accumulate into AX ---
+      auto back = [&]() {
+        if (fa.ja) HIPCHK(cqx::launch_pairs_back(fa, s));
+        if (!(scr && shared)) {
+          HIPCHK(cqx::launch_back(fa, 0, nb2_all, 0, nmat, s));
+          return;
         }
-        join_side(nst);
+        // outputs that share memory, added to in place: one after the other
+        for (int m = 0; m < nmol; ++m)
+          for (int j = 0; j < nmat; ++j)
+            HIPCHK(cqx::launch_back(fa, c->molinfo[m].nb2, c->molinfo[m + 1].nb2, j, 1, s));
       };
       // bra-range pieces of at most list_cap candidates, grouped into batches
       // of at most list_cap candidates: the quartet lists of one batch are
@@ -2045,8 +2128,9 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       size_t max_np = 1;
       for (const auto &b : batches) max_np = std::max(max_np, b.size());
       // list workspace: the per-batch tables first, then the lists
-      w.count = ws_take(c->d_count, scr, 2 * max_np, "the list counters");
-      w.psum = ws_take(c->d_psum, scr, 2 * max_np, "the list counters");
+      w.count = small ? reinterpret_cast<unsigned long long *>(w.small)
+                      : ws_take(c->d_count, scr, 2 * max_np, "the list counters");
+      w.psum = small ? w.small + nslots : ws_take(c->d_psum, scr, 2 * max_np, "the list counters");
       w.lists = ws_take(c->d_lists, scr, max_np, "the list launch table");
       w.lstart = ws_take(c->d_lstart, scr, max_np + 1, "the list launch table");
       w.quart = ws_take(c->d_quart, scr, (size_t)cap_need * qmul, "the quartet lists");
@@ -2159,13 +2243,18 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             c->stats.n_launch_eri++;
           }
       };
+      std::vector<std::pair<int, cqx_ctx::GraphSlot>> small_slots;  // launched list slots of a small build
       for (const auto &batch : batches) {
         const size_t np = batch.size();
         if (!np) continue;
         const size_t nslot = 2 * np;
         // counters cleared by a fill kernel (no memset nodes if the caller captures a graph)
-        HIPCHK(cqx::launch_zero(reinterpret_cast<double *>(w.count), nslot, s));
-        HIPCHK(cqx::launch_zero(w.psum, nslot, s));
+        if (!small) {
+          cqx::ZeroRanges z;
+          z.add(reinterpret_cast<double *>(w.count), nslot);
+          z.add(w.psum, nslot);
+          HIPCHK(cqx::launch_zero_ranges(z, s));
+        }
         std::vector<cqx::ListLaunch> lls(np);
         std::vector<long long> lstart(np + 1, 0);
         for (size_t k = 0; k < np; ++k) {
@@ -2183,6 +2272,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           LL.ket_lo = w.ket_lo + cp.coff + pc.i0;
           LL.nbra = pc.i1 - pc.i0;
           LL.ncand = pc.ncand;
+          if (small) LL.ncand_dev = w.cand + cp.coff + cp.nbra;
           LL.Bg = w.Bg;
           LL.Bm = w.Bm;
           LL.mol_boff = c->d_mol_boff.p;
@@ -2206,17 +2296,29 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           }
           lstart[k + 1] = lstart[k] + (pc.ncand + cqx::kListChunk - 1) / cqx::kListChunk;
         }
-        HIPCHK(hipMemcpyAsync(w.lists, lls.data(), sizeof(cqx::ListLaunch) * np, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(w.lstart, lstart.data(), sizeof(long long) * (np + 1), hipMemcpyHostToDevice, s));
-        HIPCHK(cqx::launch_quartet_lists(w.lists, w.lstart, (int)np, lstart[np], s));
         std::vector<unsigned long long> counts(nslot);
         std::vector<double> psum(nslot);
-        HIPCHK(hipMemcpyAsync(counts.data(), w.count, sizeof(unsigned long long) * nslot, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(psum.data(), w.psum, sizeof(double) * nslot, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
+        if (small) {
+          w.lists = ws_upload_kept(c->d_lists, c->kept_lists, nullptr, lls, s, "the list launch table");
+          w.lstart = ws_upload_kept(c->d_lstart, c->kept_lstart, nullptr, lstart, s, "the list launch table");
+          HIPCHK(cqx::launch_quartet_lists(w.lists, w.lstart, (int)np, lstart[np], s));
+          for (size_t k = 0; k < np; ++k) {
+            counts[k] = (unsigned long long)batch[k].ncand;
+            if (lls[k].out32) counts[np + k] = (unsigned long long)batch[k].ncand;
+          }
+        } else {
+          c->kept_lists.clear();
+          c->kept_lstart.clear();
+          HIPCHK(hipMemcpyAsync(w.lists, lls.data(), sizeof(cqx::ListLaunch) * np, hipMemcpyHostToDevice, s));
+          HIPCHK(hipMemcpyAsync(w.lstart, lstart.data(), sizeof(long long) * (np + 1), hipMemcpyHostToDevice, s));
+          HIPCHK(cqx::launch_quartet_lists(w.lists, w.lstart, (int)np, lstart[np], s));
+          HIPCHK(hipMemcpyAsync(counts.data(), w.count, sizeof(unsigned long long) * nslot, hipMemcpyDeviceToHost, s));
+          HIPCHK(hipMemcpyAsync(psum.data(), w.psum, sizeof(double) * nslot, hipMemcpyDeviceToHost, s));
+          HIPCHK(hipStreamSynchronize(s));
+        }
         // ERI + digestion: one launch per class pair and precision for every
         // molecule of the batch (and, with the first batch, the tile lists')
-        HIPCHK(hipEventRecord(c->ev0, s));
+        if (!small) HIPCHK(hipEventRecord(c->ev0, s));
         // autotuning times launches one by one on the context stream
         const int nst = nst_all;
         ensure_side(nst);
@@ -2234,7 +2336,8 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           cqx::EriLaunch E = eri_base(cp, pc.i0, f32);
           E.quartets = w.quart + (f32 ? cap_need : 0) + pc.seg;
           E.nq = (long long)counts[kk];
-          E.mean_prims = psum[kk] / (double)counts[kk];
+          E.mean_prims = psum[kk] / (double)counts[kk];  // (a small build has no kernel that asks for it)
+          if (small) E.nq_dev = w.count + kk;
           const int rt = route(E.la, E.lb, E.lc, E.ld);
           if (rt <= 1) {
             const int key = tune_key(E);
@@ -2269,6 +2372,11 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             apply_tuned(E);
           }
           launch_eri(E, stream_of(nlaunched++, nst));
+          c->stats.n_launch_eri++;
+          if (small) {
+            small_slots.push_back({(int)kk, {E.la, E.lb, E.lc, E.ld, E.fp32}});
+            continue;
+          }
           const double fl = class_pair_flops(E.la, E.lb, E.lc, E.ld, pure_d, psum[kk], (double)counts[kk],
                                              is_complex ? 2 : 1, nJ, nK);
           c->stats.n_quartets += (long long)counts[kk];
@@ -2278,8 +2386,8 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             c->stats.n_quartets_f32 += (long long)counts[kk];
             c->stats.flops_model_f32 += fl;
           }
-          c->stats.n_launch_eri++;
         }
+        if (small) break;  // one batch; joined with the row launches below
         join_side(nst);
         HIPCHK(hipEventRecord(c->ev1, s));
         HIPCHK(hipEventSynchronize(c->ev1));
@@ -2305,10 +2413,16 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         join_side(nst_all);
         HIPCHK(hipEventRecord(c->ev1, s));
         HIPCHK(hipMemcpyAsync(rcount.data(), c->d_rcount.p, sizeof(double) * rcount.size(), hipMemcpyDeviceToHost, s));
-        rows_back();
       }
-      back(nst_all);
-      if (!scr) {
+      std::vector<double> report(small ? 2 * nslots : 0);
+      if (small) {
+        HIPCHK(hipMemcpyAsync(report.data(), w.small, sizeof(double) * report.size(), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipMemcpyAsync(totals.data(), w.tot, sizeof(long long) * cps.size(), hipMemcpyDeviceToHost, s));
+      }
+      back();
+      if (gather) {
+        HIPCHK(hipMemcpyAsync(hbuf.data(), w.AX, sizeof(double) * gp.x, hipMemcpyDeviceToHost, s));
+      } else if (!in_place) {
         const hipMemcpyKind dk = mem == CQX_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
         for (int m = 0; m < nmol; ++m)
           for (int j = 0; j < nmat; ++j)
@@ -2316,6 +2430,28 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
                                   sizeof(double) * mnb2[m] * ew, dk, s));
       }
       HIPCHK(hipStreamSynchronize(s));
+      if (gather)
+        for (int m = 0; m < nmol; ++m)
+          for (int j = 0; j < nmat; ++j)
+            std::memcpy(list[m * nper + start + j].AX, hbuf.data() + xoff[m] + (size_t)j * mnb2[m] * ew,
+                        sizeof(double) * mnb2[m] * ew);
+      if (small) {
+        for (long long t : totals) c->stats.n_candidates += t;
+        for (const auto &sl : small_slots) {
+          const auto &G = sl.second;
+          unsigned long long n;
+          std::memcpy(&n, &report[sl.first], sizeof n);
+          const double prim = report[nslots + sl.first];
+          const double fl = class_pair_flops(G.la, G.lb, G.lc, G.ld, pure_d, prim, (double)n, is_complex ? 2 : 1, nJ, nK);
+          c->stats.n_quartets += (long long)n;
+          c->stats.n_prim_quartets_max += (long long)prim;
+          c->stats.flops_model += fl;
+          if (G.f32) {
+            c->stats.n_quartets_f32 += (long long)n;
+            c->stats.flops_model_f32 += fl;
+          }
+        }
+      }
       if (nrow) {
         float ms = 0.0f;  // with the list launches beside the row launches
         HIPCHK(hipEventElapsedTime(&ms, c->ev_r0, c->ev1));
@@ -2362,7 +2498,6 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         w.count = c->d_count.p;
         w.psum = c->d_psum.p;
         std::vector<cqx::ListLaunch> gl(ncp);
-        std::vector<long long> gidx(ncp);
         std::vector<cqx_ctx::GraphSlot> slots(2 * ncp, cqx_ctx::GraphSlot{-1, 0, 0, 0, 0});
         for (size_t k = 0; k < ncp; ++k) {
           const auto &cp = cps[k];
@@ -2402,12 +2537,9 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             LL.prim_sum32 = w.psum + ncp + k;
             slots[ncp + k] = {la_, lb_, lc_, ld_, 1};
           }
-          gidx[k] = (long long)(cp.coff + cp.nbra);
         }
         c->d_glists.upload(gl, s);
         c->d_glstart.upload(glst, s);
-        c->d_gidx.upload(gidx, s);
-        c->d_gchk.ensure(std::max<size_t>(ncp, 1));
         const int nst = c->nstreams;
         ensure_side(nst);
         HIPCHK(hipStreamSynchronize(s));  // every upload done before recording
@@ -2416,9 +2548,11 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         bool forked = false;
         try {
           front();
-          rows_front();
-          HIPCHK(cqx::launch_zero(reinterpret_cast<double *>(w.count), 2 * ncp, s));
-          HIPCHK(cqx::launch_zero(w.psum, 2 * ncp, s));
+          HIPCHK(cqx::launch_candidates_all(w.cands, (int)ncp, w.tot, s));
+          cqx::ZeroRanges z;
+          z.add(reinterpret_cast<double *>(w.count), 2 * ncp);
+          z.add(w.psum, 2 * ncp);
+          HIPCHK(cqx::launch_zero_ranges(z, s));
           HIPCHK(cqx::launch_quartet_lists(c->d_glists.p, c->d_glstart.p, (int)ncp, glst[ncp], s));
           fork_side(nst);
           forked = true;
@@ -2438,9 +2572,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           }
           join_side(nst);
           forked = false;
-          rows_back();
-          back(nst);
-          HIPCHK(cqx::launch_gather(w.cand, c->d_gidx.p, (int)ncp, c->d_gchk.p, s));
+          back();
         } catch (...) {
           if (forked)  // an unjoined side stream would leave the capture open
             for (int i = 0; i < nst - 1; ++i) {
@@ -2462,6 +2594,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         c->graph_exec = ge;
         c->graph_key = key;
         c->g_nmat = nmat;
+        c->g_x = gp.x;
         c->g_nJ = nJ;
         c->g_nK = nK;
         c->g_pure_d = pure_d;
@@ -2512,11 +2645,10 @@ int cqx_two_body_contract_noalloc(cqx_ctx *c, int screen, int ncon, const cqx_co
     int start = 0;
     while (start < nper) {
       const int nmat = group_size(list + start, nper - start, is_complex, nullptr);
-      const GroupPlan g = plan_group(c, list + start, nmat, is_complex, c->stream);
+      const GroupPlan g = plan_group(c, list + start, nmat, is_complex);
       size_t need = 0;
       auto take = [&](size_t bytes) { need = ((need + 255) & ~(size_t)255) + std::max<size_t>(bytes, 1); };
       take(g.x * sizeof(double));
-      take(nmat * sizeof(int));
       take(g.bm * sizeof(double));
       take(g.bg * sizeof(double));
       take(c->nmol * sizeof(double));
@@ -2527,10 +2659,11 @@ int cqx_two_body_contract_noalloc(cqx_ctx *c, int screen, int ncon, const cqx_co
       take(c->nmol * sizeof(cqx::MolPlanes));
       take(g.cand * sizeof(long long));
       take(g.cand * sizeof(int));
-      take(g.scan_bytes);
-      if (g.ncp) {
-        take(g.ncp * sizeof(long long));
-        take(g.ncp * sizeof(long long));
+      take(g.ncp * sizeof(cqx::CandLaunch));
+      take(g.ncp * sizeof(long long));
+      if (c->nmol > 1) {
+        take((size_t)c->nmol * nmat * sizeof(void *));
+        take((size_t)c->nmol * nmat * sizeof(void *));
       }
       need += 4096 + (g.ncp + 64) * (2 * sizeof(cqx::ListLaunch) + 64) + 256 + qmul * sizeof(Quartet);
       if (need > CQX_NOALLOC_SCRATCH_BYTES)
@@ -2558,20 +2691,19 @@ int cqx_scratch_size(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_c
   try {
     HIPCHK(hipSetDevice(c->device));
     // the buffers grow to the largest group's need; every group is sized alike
-    size_t x = 0, bm = 0, bg = 0, planes = 0, cand = 0, scan = 0, ncp = 0, nmatm = 0, pn[kNumClass] = {};
+    size_t x = 0, bm = 0, bg = 0, planes = 0, cand = 0, ncp = 0, nmatm = 0, pn[kNumClass] = {};
     long long quart = 1;
     const bool mixed = c->fp32_cut > 0.0;
     const int qmul = mixed ? 2 : 1;
     int start = 0;
     while (start < nper) {
       const int nmat = group_size(list + start, nper - start, is_complex, nullptr);
-      const GroupPlan g = plan_group(c, list + start, nmat, is_complex, c->stream);
+      const GroupPlan g = plan_group(c, list + start, nmat, is_complex);
       x = std::max(x, g.x);
       bm = std::max(bm, g.bm);
       bg = std::max(bg, g.bg);
       planes = std::max(planes, g.planes);
       cand = std::max(cand, g.cand);
-      scan = std::max(scan, g.scan_bytes);
       ncp = std::max(ncp, g.ncp);
       nmatm = std::max(nmatm, (size_t)nmat);
       for (int k = 0; k < kNumClass; ++k) pn[k] = std::max(pn[k], g.pn[k]);
@@ -2586,7 +2718,6 @@ int cqx_scratch_size(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_c
     const size_t npiece = ncp + nbra_all;
     size_t b = 0;
     b += 2 * x * sizeof(double);                     // staged densities and outputs
-    b += nmatm * sizeof(int);                        // HER flags
     b += (bm + bg + nmol) * sizeof(double);          // block norms, molecule maxima
     for (int k = 0; k < kNumClass; ++k) b += pn[k] * sizeof(double);
     b += 2 * planes * sizeof(double);                // Cartesian planes and accumulators
@@ -2601,8 +2732,8 @@ int cqx_scratch_size(cqx_ctx *c, int ncon, const cqx_contraction *list, int is_c
       }
       b += 2 * sizeof(double) * std::max<size_t>(cqx::kRowJ * pc, 1) + 3 * qmul * (ncp + 1) * sizeof(double);
     }
-    b += cand * (sizeof(long long) + sizeof(int)) + scan;
-    b += 2 * ncp * sizeof(long long);                // gathered candidate totals
+    b += cand * (sizeof(long long) + sizeof(int)) + (ncp + 1) * (sizeof(cqx::CandLaunch) + 5 * sizeof(double)) +
+         2 * sizeof(void *) * nmol * nmatm;          // candidate offsets, their launch table, totals, counters; matrix tables
     b += (size_t)quart * sizeof(Quartet);            // quartet lists
     b += npiece * (2 * sizeof(unsigned long long) + 2 * sizeof(double) + sizeof(cqx::ListLaunch) +
                    sizeof(long long)) + sizeof(long long);

@@ -66,20 +66,5 @@ struct RowLaunch {
 bool eri_row_built(int la, int lb, int lc, int ld);
 size_t eri_row_lds(int la, int lb, int lc, int ld, int fp32, int nk, int width);
 hipError_t launch_eri_row(const RowLaunch &a, hipStream_t s);
-// Coulomb planes of one class between matrix and pair order: X(second,
-// first) (non-Hermitian: X(r, c) + X(c, r)) into jx, and ja added onto the
-// accumulators (non-Hermitian: both (first, second) and (second, first))
-struct PairOrder {
-  const PairRec *pairs;
-  int npair, na, nb;
-  MolPlanes m0;
-  const MolPlanes *mols;
-  int nmol;
-  int stride[kRowJ], kind[kRowJ], idx[kRowJ], nj;
-  double *jx;
-  const double *ja;
-};
-hipError_t launch_pair_pack(const PairOrder &a, hipStream_t s);
-hipError_t launch_pair_unpack(const PairOrder &a, hipStream_t s);
 
 }  // namespace cqx

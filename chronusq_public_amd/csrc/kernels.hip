@@ -256,69 +256,6 @@ __global__ __launch_bounds__(64 * kTileListWaves) void tile_lists_kernel(const T
   }
 }
 
-// ---------------------------------------------------------------------------
-// ShellBlockNorm (direct.hpp:73-105): B(s1, s2) = max_i sum_j |X(i, j)| over
-// the (s1, s2) block.
-// ---------------------------------------------------------------------------
-__global__ void block_norm_kernel(const double *X, int nmat, int cplx, int nb, int ns,
-                                  const int *sh_bf, int bf0, const int *sh_nf, double *Bm) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long tot = (long long)nmat * ns * ns;
-  if (t >= tot) return;
-  // Bm[(s1 + s2 NS) nmat + m]
-  const int m = (int)(t % nmat);
-  const int rem = (int)(t / nmat);
-  const int s1 = rem % ns, s2 = rem / ns;
-  const size_t nb2 = (size_t)nb * nb;
-  const double *Xm = X + (size_t)m * nb2 * (cplx ? 2 : 1);
-  double mx = 0.0;
-  for (int i = 0; i < sh_nf[s1]; ++i) {
-    double row = 0.0;
-    for (int j = 0; j < sh_nf[s2]; ++j) {
-      const size_t idx = (sh_bf[s1] - bf0 + i) + (size_t)(sh_bf[s2] - bf0 + j) * nb;
-      row += cplx ? hypot(Xm[2 * idx], Xm[2 * idx + 1]) : fabs(Xm[idx]);
-    }
-    mx = fmax(mx, row);
-  }
-  Bm[t] = mx;
-}
-
-__global__ void pair_norm_kernel(const PairScr *pairs, int npair, const double *Bg, const double *Bm,
-                                 const long long *mol_boff, const int *mol_ns, int nmat, double *pn) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npair) return;
-  const PairScr P = pairs[i];
-  const int s1 = (int)(P.s12 & 0xFFFFu), s2 = (int)(P.s12 >> 16);
-  const size_t b = (size_t)mol_boff[P.mol] + s1 + (size_t)s2 * mol_ns[P.mol];
-  pn[(size_t)i * (nmat + 1)] = Bg[b];
-  for (int m = 0; m < nmat; ++m) pn[(size_t)i * (nmat + 1) + 1 + m] = Bm[b * nmat + m];
-}
-
-__global__ void block_norm_finish_kernel(int nmat, int ns, const double *Bm, double *Bg) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)ns * ns) return;
-  const int k = (int)(t % ns), l = (int)(t / ns);
-  // per-matrix norms are already symmetrised (block_norm_symm_kernel)
-  double g = 0.0;
-  for (int m = 0; m < nmat; ++m) g = fmax(g, Bm[(k + (size_t)l * ns) * nmat + m]);
-  Bg[k + (size_t)l * ns] = g;
-}
-
-__global__ void block_norm_symm_kernel(int nmat, int ns, const int *her, double *Bm) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)nmat * ns * ns) return;
-  const int m = (int)(t % nmat);
-  if (her[m]) return;
-  const int rem = (int)(t / nmat);
-  const int k = rem % ns, l = rem / ns;
-  if (k <= l) return;
-  // symmetrised for non-Hermitian X, direct.hpp:1537-1545
-  double *B1 = Bm + (k + (size_t)l * ns) * nmat + m, *B2 = Bm + (l + (size_t)k * ns) * nmat + m;
-  const double mx = fmax(*B1, *B2);
-  *B1 = mx;
-  *B2 = mx;
-}
-
 __device__ __forceinline__ int sph_off(int l) {
   // sum_{k<l} (2k+1) ncart(k): 0, 1, 10, 40, 110
   const int off[5] = {0, 1, 10, 40, 110};
@@ -363,10 +300,9 @@ __global__ void to_cart_kernel(CartMap M, const double *X, int cplx, double *Pre
   if (Pim) Pim[t * ps] = im;
 }
 
-// blockIdx.y: matrix of a batch of equal ones, sa / sx doubles apart
-__global__ void from_cart_kernel(CartMap M, const double *Are, const double *Aim, int ps,
-                                 int her, int cplx, double *AX, size_t sa, size_t sx) {
-  Are += blockIdx.y * sa;
+// blockIdx.y: matrix of a batch of equal real ones, sa / sx doubles apart
+__global__ void from_cart_kernel(CartMap M, const double *A, int her, double *AX, size_t sa, size_t sx) {
+  A += blockIdx.y * sa;
   AX += blockIdx.y * sx;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long long)M.nb * M.nb) return;
@@ -374,59 +310,18 @@ __global__ void from_cart_kernel(CartMap M, const double *Are, const double *Aim
   const int sm = M.bf_shell[mu], cm = M.bf_comp[mu];
   const int sn = M.bf_shell[nu], cn = M.bf_comp[nu];
   const int ncm = ncart_d(M.sh_l[sm]), ncn = ncart_d(M.sh_l[sn]);
-  double a_re = 0.0, a_im = 0.0, b_re = 0.0, b_im = 0.0;
+  double a = 0.0, b = 0.0;
   for (int i = 0; i < ncm; ++i) {
     const double ti = tcoef(M, sm, i, cm);
     if (ti == 0.0) continue;
     for (int j = 0; j < ncn; ++j) {
       const double tj = tcoef(M, sn, j, cn);
       if (tj == 0.0) continue;
-      const size_t ij = (M.sh_bfc[sm] - M.bfc0 + i) + (size_t)(M.sh_bfc[sn] - M.bfc0 + j) * M.nbc;
-      const size_t ji = (M.sh_bfc[sn] - M.bfc0 + j) + (size_t)(M.sh_bfc[sm] - M.bfc0 + i) * M.nbc;
-      a_re += ti * tj * Are[ij * ps];
-      b_re += ti * tj * Are[ji * ps];
-      if (Aim) {
-        a_im += ti * tj * Aim[ij * ps];
-        b_im += ti * tj * Aim[ji * ps];
-      }
+      a += ti * tj * A[(M.sh_bfc[sm] - M.bfc0 + i) + (size_t)(M.sh_bfc[sn] - M.bfc0 + j) * M.nbc];
+      b += ti * tj * A[(M.sh_bfc[sn] - M.bfc0 + j) + (size_t)(M.sh_bfc[sm] - M.bfc0 + i) * M.nbc];
     }
   }
-  double re, im;
-  if (her) {  // 1/2 (A + A^H), direct.hpp:2040-2049
-    re = 0.5 * (a_re + b_re);
-    im = 0.5 * (a_im - b_im);
-  } else {    // 1/2 A, direct.hpp:2051-2062
-    re = 0.5 * a_re;
-    im = 0.5 * a_im;
-  }
-  if (cplx) {
-    AX[2 * t] += re;
-    AX[2 * t + 1] += im;
-  } else {
-    AX[t] += re;
-  }
-}
-
-// max of each molecule's block of global block norms (one block per molecule)
-__global__ void mol_max_kernel(const double *Bg, const long long *mol_boff, const int *mol_ns, double *out) {
-  const int m = blockIdx.x;
-  const long long n = (long long)mol_ns[m] * mol_ns[m];
-  const double *B = Bg + mol_boff[m];
-  double v = 0.0;
-  for (long long i = threadIdx.x; i < n; i += blockDim.x) v = fmax(v, B[i]);
-  __shared__ double red[256];
-  red[threadIdx.x] = v;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[m] = red[0];
-}
-
-__global__ void gather_kernel(const long long *src, const long long *idx, int n, long long *dst) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[idx[i]];
+  AX[t] += her ? 0.5 * (a + b) : 0.5 * a;  // 1/2 (A + A^H), direct.hpp:2040-2049; 1/2 A, :2051-2062
 }
 
 __global__ void zero_kernel(double *p, size_t n) {
@@ -458,39 +353,10 @@ hipError_t launch_quartet_lists(const ListLaunch *lists, const long long *start,
   return hipGetLastError();
 }
 
-hipError_t launch_pair_norms(const PairScr *pairs, int npair, const double *Bg, const double *Bm,
-                             const long long *mol_boff, const int *mol_ns, int nmat, double *pn,
-                             hipStream_t s) {
-  if (npair <= 0) return hipSuccess;
-  hipLaunchKernelGGL(pair_norm_kernel, dim3(nblocks(npair, 256)), dim3(256), 0, s, pairs, npair, Bg, Bm,
-                     mol_boff, mol_ns, nmat, pn);
-  return hipGetLastError();
-}
-
-hipError_t launch_block_norms(const double *X, int nmat, int is_complex, const int *her, int nb,
-                              int ns, const int *sh_bf, int bf0, const int *sh_nf, double *Bm, double *Bg,
-                              hipStream_t s) {
-  const long long n1 = (long long)nmat * ns * ns;
-  hipLaunchKernelGGL(block_norm_kernel, dim3(nblocks(n1, 256)), dim3(256), 0, s, X, nmat,
-                     is_complex, nb, ns, sh_bf, bf0, sh_nf, Bm);
-  hipLaunchKernelGGL(block_norm_symm_kernel, dim3(nblocks(n1, 256)), dim3(256), 0, s, nmat, ns,
-                     her, Bm);
-  hipLaunchKernelGGL(block_norm_finish_kernel, dim3(nblocks((long long)ns * ns, 256)), dim3(256),
-                     0, s, nmat, ns, Bm, Bg);
-  return hipGetLastError();
-}
-
 hipError_t launch_to_cart(const CartMap &m, const double *X, int is_complex, double *pre,
                           double *pim, int ps, hipStream_t s) {
   hipLaunchKernelGGL(to_cart_kernel, dim3(nblocks((long long)m.nbc * m.nbc, 256)), dim3(256), 0,
                      s, m, X, is_complex, pre, pim, ps);
-  return hipGetLastError();
-}
-
-hipError_t launch_from_cart(const CartMap &m, const double *are, const double *aim, int ps, int her,
-                            int is_complex, double *AX, hipStream_t s) {
-  hipLaunchKernelGGL(from_cart_kernel, dim3(nblocks((long long)m.nb * m.nb, 256)), dim3(256), 0,
-                     s, m, are, aim, ps, her, is_complex, AX, (size_t)0, (size_t)0);
   return hipGetLastError();
 }
 
@@ -499,21 +365,8 @@ hipError_t launch_from_cart_many(const CartMap &m, const double *a, size_t sa, i
   for (size_t k = 0; k < n; k += 65535) {
     const unsigned ny = (unsigned)std::min<size_t>(65535, n - k);
     hipLaunchKernelGGL(from_cart_kernel, dim3(nblocks((long long)m.nb * m.nb, 256), ny), dim3(256), 0, s, m, a + k * sa,
-                       (const double *)nullptr, 1, her, 0, AX + k * sx, sa, sx);
+                       her, AX + k * sx, sa, sx);
   }
-  return hipGetLastError();
-}
-
-hipError_t launch_mol_max(const double *Bg, const long long *mol_boff, const int *mol_ns, int nmol,
-                          double *out, hipStream_t s) {
-  if (nmol <= 0) return hipSuccess;
-  hipLaunchKernelGGL(mol_max_kernel, dim3(nmol), dim3(256), 0, s, Bg, mol_boff, mol_ns, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_gather(const long long *src, const long long *idx, int n, long long *dst, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(gather_kernel, dim3(nblocks(n, 256)), dim3(256), 0, s, src, idx, n, dst);
   return hipGetLastError();
 }
 

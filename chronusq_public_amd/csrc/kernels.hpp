@@ -128,8 +128,6 @@ struct ListLaunch {
 // 1024-candidate chunks [start[k], start[k + 1]) of a common chunk space
 // (start: nlist + 1 entries on the device, nchunk = start[nlist]).
 constexpr int kListChunk = 1024;
-// dst[i] = src[idx[i]], i < n (one launch; reads back counters in one copy)
-hipError_t launch_gather(const long long *src, const long long *idx, int n, long long *dst, hipStream_t s);
 hipError_t launch_quartet_lists(const ListLaunch *lists, const long long *start, int nlist, long long nchunk,
                                 hipStream_t s);
 // Tile lists of the tile class pairs of a build: sub-block t of a list
@@ -189,15 +187,9 @@ hipError_t launch_eri_tile(const TileEriLaunch &a, hipStream_t s);
 // tile kernel)
 int tile_acc_doubles(int la, int lb, int lc, int ld, const PlaneSet &ps);
 
-// pn[i (nmat + 1) + k] = block norm of pair i's own shells (k = 0 global,
-// k = 1 + m matrix m)
-hipError_t launch_pair_norms(const PairScr *pairs, int npair, const double *Bg, const double *Bm,
-                             const long long *mol_boff, const int *mol_ns, int nmat, double *pn,
-                             hipStream_t s);
-
 // Candidate kets of every bra pair of one class pair: off[i + 1] - off[i]
 // kets starting at klo[i] (the bra's molecule's first ket), off an
-// inclusive prefix (off[0] = 0).  tmp == nullptr queries tmp_bytes.
+// inclusive prefix (off[0] = 0).
 struct CandLaunch {
   const PairRec *bra, *ket;
   int nbra;
@@ -209,17 +201,6 @@ struct CandLaunch {
   long long *off;          // nbra + 1
   int *klo;                // nbra
 };
-hipError_t launch_candidates(const CandLaunch &a, void *tmp, size_t &tmp_bytes, hipStream_t s);
-
-// Shell-block infinity norms (max absolute row sum) of nmat spherical
-// matrices; symmetrised for non-Hermitian ones; global max over matrices.
-hipError_t launch_block_norms(const double *X, int nmat, int is_complex,
-                              const int *her, int nb, int ns,
-                              const int *sh_bf, int bf0, const int *sh_nf,
-                              double *Bm, double *Bg, hipStream_t s);
-// out[m] = max of molecule m's global block norms
-hipError_t launch_mol_max(const double *Bg, const long long *mol_boff, const int *mol_ns, int nmol,
-                          double *out, hipStream_t s);
 
 // Cartesian <-> pure transforms of whole matrices.
 struct CartMap {
@@ -242,11 +223,8 @@ struct CartMap {
 // with interleave stride ps (plane pointers already offset to their slot)
 hipError_t launch_to_cart(const CartMap &m, const double *X, int is_complex,
                           double *plane_re, double *plane_im, int ps, hipStream_t s);
-// AX += finalize(T^T A T): her = 1 gives 1/2 (A + A^H), her = 0 gives 1/2 A;
-// A_im may be null (real accumulator only); planes interleaved with stride ps.
-hipError_t launch_from_cart(const CartMap &m, const double *A_re, const double *A_im, int ps,
-                            int her, int is_complex, double *AX, hipStream_t s);
-// n real matrices, sa / sx doubles apart, in one launch
+// AX += finalize(T^T A T) for n real matrices, sa / sx doubles apart, in one
+// launch: her = 1 gives 1/2 (A + A^T), her = 0 gives 1/2 A
 hipError_t launch_from_cart_many(const CartMap &m, const double *a, size_t sa, int her, double *AX, size_t sx,
                                  size_t n, hipStream_t s);
 
