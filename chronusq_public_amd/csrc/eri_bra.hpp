@@ -29,17 +29,17 @@ using GlobalDouble = __attribute__((address_space(1))) double;
 
 namespace {
 
-// Add to I the primitive quartets of a bra pair that is the same for the
-// whole wave (bp; its records come through the scalar cache) with the ket's
+// Add to I the primitive quartets of primitives [i0, i1) of a bra pair that
+// is the same for the whole wave (bp; its records come through the scalar cache) with the ket's
 // primitive pairs g, g + G, ... below nk, each held in registers while the
 // bra's primitives pass by.
 template <int LA, int LB, int LC, int LD, class R>
 __device__ __forceinline__ void eval_bra(const PrimPair *prims, const PrimC32 *pc32, const R *__restrict__ rysn,
-                                         ConstPtr<PairRec> bp, const double (&Cc)[3], const double (&CDc)[3],
+                                         ConstPtr<PairRec> bp, int i0, int i1, const double (&Cc)[3], const double (&CDc)[3],
                                          int koff, int nk, int g, int G, R (&I)[Cls<LA, LB, LC, LD>::NC]) {
   using K = Cls<LA, LB, LC, LD>;
   constexpr bool F32 = std::is_same<R, float>::value;
-  const int boff = bp->pp_off, nb = bp->npp;
+  const int boff = bp->pp_off;
   R AB[3], CD[3], AC[3];
   double Ac[3];
 #pragma unroll
@@ -73,7 +73,7 @@ __device__ __forceinline__ void eval_bra(const PrimPair *prims, const PrimC32 *p
         QC[d] = B.P[d] - Cc[d];
       }
     }
-    for (int i = 0; i < nb; ++i) {
+    for (int i = i0; i < i1; ++i) {
       R ap, rp, PA[3], PQ[3], pref;
       R r, rpq;
       if constexpr (F32) {

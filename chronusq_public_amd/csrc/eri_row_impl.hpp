@@ -18,18 +18,21 @@
 // neighbouring lanes hold neighbouring doubles.
 //
 // Each block screens its own kets (no quartet list, no host round trip) and
-// sorts the survivors into two bins by contraction length, the long ones
-// with more lanes per ket, so that a wave's lanes have similar loops.
+// sorts the survivors by their primitive pairs, so that the lanes of a wave
+// run loops of one length.  With two bins (contraction products up to 8 and
+// beyond) half of the lanes idled: 6-31G(d) carbon pairs have 1, 3 or 6 in
+// the first and 9, 18 or 36 in the second.  Measured with the bins and
+// sorted (ms a build): C40H82 / 6-31G(d) 32.7 -> 28.5, mixed 29.2 -> 25.0, 32
+// water clusters batched, mixed, 34.0 -> 28.5, (H2O)4 / cc-pVDZ 0.79 -> 0.61,
+// non-Hermitian complex (H2O)7 1.63 -> 1.32.
 //
-// Measured against the quartet-list build (ms a build): C40H82 / 6-31G(d)
-// FP64 90.5 -> 36.9, mixed 71.5 -> 30.8; 32 water clusters batched, mixed,
-// 75 -> 38; GHF (H2O)16 / cc-pVDZ 12.8 -> 9.4; non-Hermitian complex (H2O)7
-// 3.2 -> 2.0; (H2O)4 1.38 -> 1.10.
+// Measured against the quartet-list build (ms a build, two bins): C40H82
+// 90.5 -> 36.9, mixed 71.5 -> 30.8; the batch 75 -> 38; GHF (H2O)16 / cc-pVDZ
+// 12.8 -> 9.4; (H2O)7 3.2 -> 2.0; (H2O)4 1.38 -> 1.10.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#include "digest.hpp"
 #include <mutex>
 
 #include "digest.hpp"
@@ -42,20 +45,20 @@ namespace cqx {
 
 namespace {
 
-// contraction-length product above which a ket goes to the long bin
-constexpr int kRowLongKet = 8;
+// Buckets of the surviving kets by their primitive pairs: exact up to 32,
+// then in fours, the last one open.  bucket_most: the most primitive pairs of
+// a bucket (of the open one a stand-in: it takes the most lanes anyway).
+constexpr int kRowBuckets = 64;
+__device__ __forceinline__ int row_bucket(int npp) {
+  return npp <= 32 ? max(npp, 1) - 1 : min(32 + (npp - 33) / 4, kRowBuckets - 1);
+}
+__device__ __forceinline__ int bucket_most(int k) { return k < 32 ? k + 1 : 36 + 4 * (k - 32); }
 
 // sum over the wave, in every lane
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   return v;
-}
-
-__device__ __forceinline__ int pow2_at_least(int n) {
-  int p = 1;
-  while (p < n) p *= 2;
-  return p;
 }
 
 // The four exchange updates of one quartet in row form: with rows Xa = X(a, :)
@@ -149,9 +152,10 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
   constexpr int NROW = K::NCA + K::NCB, NAB = K::NCA * K::NCB, NCD = K::NCC * K::NCD;
   extern __shared__ double s_rows[];
   __shared__ R s_tab[rys_tab_len(K::NR)];
-  __shared__ unsigned s_queue[kRowChunk];  // short kets from the front, long ones from the back
+  __shared__ unsigned s_queue[kRowChunk];  // surviving kets, most primitive pairs first
+  __shared__ int s_hist[kRowBuckets];
   __shared__ double s_jab[kRowJ * NAB];
-  __shared__ int s_n[2], s_next;
+  __shared__ int s_next;
   __shared__ unsigned long long s_tot[2];
   __shared__ double s_psum;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -191,22 +195,25 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
       if (a.fp32 && !(Qi * as_const(a.kscr + (j1 - 1))->Q < a.cut32)) continue;
     }
     __syncthreads();  // the previous item's rows, queue and sums have been read
-    if (tid == 0) {
-      s_n[0] = s_n[1] = 0;
-      s_next = 0;
-    }
+    if (tid < kRowBuckets) s_hist[tid] = 0;
+    if (tid == 0) s_next = 0;
     __syncthreads();
     const PairScr P = a.bscr[i];
     const ScreenArgs sa{a.Bg, a.Bm, a.mol_boff, a.mol_ns, a.nmat, a.thresh, a.screen};
     int ncand = 0;
     double psum = 0.0;
-    for (int t = tid; t < kRowChunk; t += kRowThreads) {
-      const int j = j0 + t;
+    constexpr int kPer = kRowChunk / kRowThreads;
+    unsigned mine[kPer];  // ket, contractions
+    int place[kPer];      // bucket and rank in it (< 0: none)
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int t = tid + u * kRowThreads, j = j0 + t;
       bool pass = false, cand = false;
       unsigned mask = 0;
-      int kk = 0;
+      int kk = 0, npp = 0;
       if (j < j1) {
         const PairScr Q = a.kscr[j];
+        npp = a.ket[j].npp;
         const double qq = P.Q * Q.Q;
         kk = Q.kk;
         const bool lo32 = a.cut32 > 0.0 && qq < a.cut32;
@@ -217,19 +224,13 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
         }
       }
       ncand += __popcll(__ballot(cand));
-      if (pass) psum += (double)P.kk * (double)kk;
-      const bool lng = kk > kRowLongKet;
-      const unsigned long long b0 = __ballot(pass && !lng), b1 = __ballot(pass && lng);
-      int p0 = 0, p1 = 0;
-      if (lane == 0) {
-        if (b0) p0 = atomicAdd(&s_n[0], (int)__popcll(b0));
-        if (b1) p1 = atomicAdd(&s_n[1], (int)__popcll(b1));
+      mine[u] = (unsigned)t | (mask << 16);
+      place[u] = -1;
+      if (pass) {
+        psum += (double)P.kk * (double)kk;
+        const int b = row_bucket(npp);
+        place[u] = b | (atomicAdd(&s_hist[b], 1) << 8);
       }
-      p0 = __shfl(p0, 0);
-      p1 = __shfl(p1, 0);
-      const unsigned long long below = (1ull << lane) - 1ull;
-      if (pass && !lng) s_queue[p0 + __popcll(b0 & below)] = (unsigned)t | (mask << 16);
-      if (pass && lng) s_queue[kRowChunk - 1 - (p1 + __popcll(b1 & below))] = (unsigned)t | (mask << 16);
     }
     psum = wave_sum(psum);
     if (lane == 0) {
@@ -237,9 +238,46 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
       if (psum != 0.0) unsafeAtomicAdd(&s_psum, psum);
     }
     __syncthreads();
-    const int n0 = s_n[0], n1 = s_n[1];
-    if (n0 + n1 == 0) continue;
-    if (tid == 0) s_tot[0] += (unsigned long long)(n0 + n1);
+    // every wave for itself: kets in the buckets from lane's own up (the
+    // queue is in descending order), and the primitive pairs of all
+    const int cnt = s_hist[lane], most = bucket_most(lane);
+    int upto = cnt, work = cnt * most;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_down(upto, o);
+      if (lane + o < 64) upto += v;
+      work += __shfl_xor(work, o);
+    }
+    const int n = __builtin_amdgcn_readfirstlane(upto);
+    if (n == 0) continue;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int first = __shfl(upto - cnt, place[u] & (kRowBuckets - 1));
+      if (place[u] >= 0) s_queue[first + (place[u] >> 8)] = mine[u];
+    }
+    if (tid == 0) s_tot[0] += (unsigned long long)n;
+    // Lanes per ket: a lane takes at most `turns` primitive pairs, so that no
+    // ket outlasts an even share of the block's work (one lane each in a full
+    // chunk, whose digestion then uses every lane; up to 64 where a bra has a
+    // handful of kets); kets [end[l + 1], end[l]) of the queue get 2^l lanes.
+    work = __builtin_amdgcn_readfirstlane(work);
+    const int turns = max(1, work / kRowThreads);
+    int end[8], nunit = 0;
+    end[0] = n;
+    end[7] = 0;
+#pragma unroll
+    for (int l = 1; l < 7; ++l) {
+      const unsigned long long more = __ballot(most > (turns << (l - 1)));
+      end[l] = more ? __builtin_amdgcn_readlane(upto, (int)__builtin_ctzll(more)) : 0;
+    }
+#pragma unroll
+    for (int l = 0; l < 7; ++l) nunit += (((end[l] - end[l + 1]) << l) + 63) >> 6;
+    // with fewer units than waves, each unit's bra primitives are dealt over
+    // several waves (the digestion is linear in the integrals), two or more
+    // each: a chain of 64 bra primitives is 8 long in a small molecule
+    const int nb = bp->npp;
+    int nsplit = 1;
+    while (2 * nsplit * nunit <= kRowThreads / 64 && nb >= 4 * nsplit) nsplit *= 2;
     // the molecule's planes; density rows in, exchange rows cleared
     const bool one = a.nmol == 1;
     const ConstPtr<MolPlanes> mp = as_const(a.mols + (one ? 0 : mol));
@@ -265,26 +303,28 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
     }
     for (int e = tid; e < a.nj * NAB; e += kRowThreads) s_jab[e] = 0.0;
     __syncthreads();
-    // lanes per ket of each bin: enough for the block's lanes when there are
-    // few kets, and for at most about 128 primitive quartets per lane
-    const int nb = bp->npp;
-    int g0 = 1, g1 = 4;
-    while (g0 < 8 && (n0 * g0 < kRowThreads || nb * (kRowLongKet / g0) > 128)) g0 *= 2;
-    while (g1 < 16 && (n1 * g1 < kRowThreads || nb * (32 / g1) > 128)) g1 *= 2;
-    const int ng1 = (n1 * g1 + 63) >> 6, ng0 = (n0 * g0 + 63) >> 6;
     const int pa = bp->a, pb = bp->b;
     const double bra_scale = 0.5 * (pa == pb ? 1.0 : 2.0);
     for (;;) {
       int grp = 0;
       if (lane == 0) grp = atomicAdd(&s_next, 1);
       grp = __builtin_amdgcn_readfirstlane(grp);
-      if (grp >= ng0 + ng1) break;
-      const bool lng = grp < ng1;
-      const int G = lng ? g1 : g0, nbin = lng ? n1 : n0;
-      const int lg = __builtin_ctz(G);
-      const int slot = ((lng ? grp : grp - ng1) << (6 - lg)) + (lane >> lg), g = lane & (G - 1);
-      const bool valid = slot < nbin;
-      const unsigned q = valid ? s_queue[lng ? kRowChunk - 1 - slot : slot] : 0u;
+      if (grp >= nunit * nsplit) break;
+      const int part = grp / nunit;
+      int unit = grp - part * nunit, lg = 0, from = 0, to = 0;
+#pragma unroll
+      for (int l = 6; l >= 0; --l) {
+        const int m = (((end[l] - end[l + 1]) << l) + 63) >> 6;
+        if (unit >= 0 && unit < m) {
+          lg = l;
+          from = end[l + 1] + (unit << (6 - l));
+          to = end[l];
+        }
+        unit -= m;
+      }
+      const int G = 1 << lg, slot = from + (lane >> lg), g = lane & (G - 1);
+      const bool valid = slot < to;
+      const unsigned q = valid ? s_queue[slot] : 0u;
       const int j = j0 + (int)(q & 0xFFFFu);
       const unsigned mask = q >> 16;
       int koff = 0, nkp = 0, c = 0, d = 0, fc = 0, fd = 0;
@@ -306,7 +346,8 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
       R I[K::NC];
 #pragma unroll
       for (int o = 0; o < K::NC; ++o) I[o] = 0;
-      eval_bra<LA, LB, LC, LD, R>(a.prims, a.primc32, s_tab, bp, Cc, CD, koff, nkp, g, G, I);
+      eval_bra<LA, LB, LC, LD, R>(a.prims, a.primc32, s_tab, bp, nb * part / nsplit, nb * (part + 1) / nsplit, Cc, CD,
+                                  koff, nkp, g, G, I);
       for (int off = G >> 1; off > 0; off >>= 1) {
 #pragma unroll
         for (int o = 0; o < K::NC; ++o) I[o] += __shfl_xor(I[o], off);
@@ -403,7 +444,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
 // rows (exchange, and density)
 template <class K, class R>
 size_t row_lds(int nk, int width, int sets) {
-  const size_t fixed = sizeof(R) * rys_tab_len(K::NR) + 4 * kRowChunk + 8 * kRowJ * K::NCA * K::NCB + 256;
+  const size_t fixed = sizeof(R) * rys_tab_len(K::NR) + 4 * (kRowChunk + kRowBuckets) + 8 * kRowJ * K::NCA * K::NCB + 256;
   return fixed + (size_t)sets * nk * (K::NCA + K::NCB) * width * sizeof(double);
 }
 
