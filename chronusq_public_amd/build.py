@@ -5,6 +5,7 @@ integrals, the SCF driver) and csrc/*.hip (device kernels); linked against
 rocBLAS and rocSOLVER from the ROCm install.  The Rys table (csrc/rys_table.bin, written by
 csrc/gen_rys_table.py) is embedded as a C array.
 """
+import math
 import os
 import subprocess
 import sys
@@ -37,16 +38,56 @@ def rys_powers(tab):
         cheb[k, 1:] = 2 * cheb[k - 1, :-1]
         cheb[k] -= cheb[k - 2]
     scale = np.longdouble(2) ** np.arange(n)
-    return (tab.reshape(-1, n).astype(np.longdouble) @ cheb * scale).astype(np.float64).ravel()
+    return (tab.reshape(-1, n).astype(np.longdouble) @ cheb * scale).ravel()
 
 
-def write_rys_inc():
-    tab = rys_powers(np.fromfile(os.path.join(CSRC, "rys_table.bin"), dtype="<f8"))
-    path = os.path.join(CSRC, "rys_table_data.inc")
+def rys_halves(tab, nmax, ncoef):
+    """The sections of 1..nmax roots on half intervals of T: series in
+    v = 4 (T - (m/2 + 1/4)) cut after ncoef Chebyshev terms, in powers of
+    t = v / 4, laid out [half interval][power][value]; extended precision."""
+    n = 14  # CQX_RYS_NCOEF
+    L = np.longdouble
+    cheb = np.zeros((n, n), dtype=L)  # powers of each Chebyshev polynomial
+    cheb[0, 0] = cheb[1, 1] = 1
+    for k in range(2, n):
+        cheb[k, 1:] = 2 * cheb[k - 1, :-1]
+        cheb[k] -= cheb[k - 2]
+    inv = np.eye(n, dtype=L)  # Chebyshev series of each power
+    for k in range(n):
+        for j in range(k):
+            inv[k] -= cheb[k, j] * inv[j]
+        inv[k] /= cheb[k, k]
+    keep = np.diag((np.arange(n) < ncoef).astype(L))
+    out, off = [], 0
+    for roots in range(1, nmax + 1):
+        m, nval = 34 + 6 * roots, 2 * roots
+        powers = tab[off:off + m * nval * n].reshape(m * nval, n).astype(L) @ cheb  # of u
+        off += m * nval * n
+        half = []
+        for a in (-0.5, 0.5):  # u = a + v / 2
+            shift = np.zeros((n, n), dtype=L)
+            for k in range(n):
+                for j in range(k + 1):
+                    shift[k, j] = math.comb(k, j) * L(a) ** (k - j) * L(0.5) ** j
+            p = (powers @ shift @ inv @ keep @ cheb) * L(4) ** np.arange(n)
+            half.append(p[:, :ncoef].reshape(m, nval, ncoef).transpose(0, 2, 1))
+        out.append(np.stack(half, axis=1).ravel())
+    return np.concatenate(out)
+
+
+def _write_values(name, tab):
+    path = os.path.join(CSRC, name)
     with open(path, "w") as f:
         for i in range(0, tab.size, 4):
             f.write(", ".join(float(v).hex() for v in tab[i:i + 4]) + ",\n")
     return path
+
+
+def write_rys_inc():
+    raw = np.fromfile(os.path.join(CSRC, "rys_table.bin"), dtype="<f8")
+    _write_values("rys_half_data.inc", rys_halves(raw, 2, 11).astype(np.float64))
+    _write_values("rys_half32_data.inc", rys_halves(raw, 3, 6).astype(np.float32))
+    return _write_values("rys_table_data.inc", rys_powers(raw).astype(np.float64))
 
 
 # the sources of the ERI + digestion launches of a Fock build: the kernels,
@@ -63,7 +104,7 @@ def source_digest():
     import hashlib
     h = hashlib.sha256()
     for f in sorted(os.listdir(CSRC)):
-        if not f.startswith(KERNEL_SOURCES) or f == "rys_table_data.inc":
+        if not f.startswith(KERNEL_SOURCES) or f.endswith("_data.inc"):
             continue
         h.update(f.encode())
         with open(os.path.join(CSRC, f), "rb") as fh:

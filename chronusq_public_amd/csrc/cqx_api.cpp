@@ -33,6 +33,13 @@ namespace {
 const double kRysTable[] = {
 #include "rys_table_data.inc"
 };
+// the row kernels' forms of its first sections (RysRow)
+const double kRysHalf[] = {
+#include "rys_half_data.inc"
+};
+const float kRysHalf32[] = {
+#include "rys_half32_data.inc"
+};
 
 thread_local std::string g_error;  // error of the last failing call of this thread
 
@@ -193,8 +200,8 @@ struct cqx_ctx {
   // accumulators and outputs
   DevBuf<int> d_shell_atom;
   DevBuf<double> d_gX, d_gacc, d_gAX;
-  DevBuf<double> d_rys, d_sph;
-  DevBuf<float> d_rys32;
+  DevBuf<double> d_rys, d_rys_half, d_sph;
+  DevBuf<float> d_rys32, d_rys32_half;
   DevBuf<int> d_cart_shell, d_cart_comp, d_sh_bf, d_sh_bfc, d_sh_l, d_sh_pure, d_sh_nf,
       d_bf_shell, d_bf_comp;
   cqx::CartMap cmap{};
@@ -927,6 +934,10 @@ void init_ctx(cqx_ctx *c, const cqx::Basis &basis, double thresh, int device) {
   c->d_rys.upload(rys, c->stream);
   std::vector<float> rys32(rys.begin(), rys.end());
   c->d_rys32.upload(rys32, c->stream);
+  const std::vector<double> half(std::begin(kRysHalf), std::end(kRysHalf));
+  c->d_rys_half.upload(half, c->stream);
+  const std::vector<float> half32(std::begin(kRysHalf32), std::end(kRysHalf32));
+  c->d_rys32_half.upload(half32, c->stream);
   HIPCHK(hipStreamSynchronize(c->stream));
   setup_device_maps(c);
 }
@@ -1889,7 +1900,8 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             R.prims = c->d_prims.p;
             R.primc32 = c->d_primc32.p;
             R.rys = c->d_rys.p;
-            R.rys32 = c->d_rys32.p;
+            R.rys_half = c->d_rys_half.p;
+            R.rys32_half = c->d_rys32_half.p;
             R.m0 = mp[0];
             R.mols = w.molplanes;
             R.nmol = nmol;

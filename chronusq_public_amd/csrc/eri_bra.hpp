@@ -33,7 +33,7 @@ namespace {
 // is the same for the whole wave (bp; its records come through the scalar cache) with the ket's
 // primitive pairs g, g + G, ... below nk, each held in registers while the
 // bra's primitives pass by.
-template <int LA, int LB, int LC, int LD, class R>
+template <int LA, int LB, int LC, int LD, class R, bool ROOM>
 __device__ __forceinline__ void eval_bra(const PrimPair *prims, const PrimC32 *pc32, const R *__restrict__ rysn,
                                          ConstPtr<PairRec> bp, int i0, int i1, const double (&Cc)[3], const double (&CDc)[3],
                                          int koff, int nk, int g, int G, R (&I)[Cls<LA, LB, LC, LD>::NC]) {
@@ -105,7 +105,7 @@ __device__ __forceinline__ void eval_bra(const PrimPair *prims, const PrimC32 *p
       const R rho = ap * bqr;
       const R T = rho * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]);
       R x[K::NR], w[K::NR];
-      rys_roots_sec<K::NR, R>(T, rysn, x, w);
+      rys_roots_row<K::NR, R, K::NC == 1, ROOM>(T, rysn, x, w);
       if constexpr (K::NC == 1) {
         I[0] = fma(pref, w[0], I[0]);
       } else {

@@ -41,8 +41,8 @@ struct RowLaunch {
   int fp32;
   const PrimPair *prims;
   const PrimC32 *primc32;
-  const double *rys;
-  const float *rys32;
+  const double *rys, *rys_half;  // the Rys table, and its forms for the row kernels (RysRow)
+  const float *rys32_half;
   MolPlanes m0;
   const MolPlanes *mols;
   int nmol;

@@ -33,6 +33,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "digest.hpp"
@@ -141,17 +142,28 @@ __device__ __forceinline__ void digest_rows(const double (&I)[K::NC], const X &x
 // exchange rows ([plane][NA + NB][width]), then, with XL, the density rows;
 // without XL the density is read from its planes in global memory (many
 // planes, whose density rows would not fit beside the exchange rows).
+// Most threads of a block (256 where a lane takes more than 256 registers),
+// and wavefronts per SIMD asked of the compiler: six for the classes that fit
+// 80 registers (C40H82 / 6-31G(d), ms a launch: (ss|ss) 2.72 -> 2.27, (ps|ss)
+// 3.67 -> 3.40 for the compiler's own five; five for (ps|ps) spill, 1.89 ->
+// 2.37).
 template <class K>
 constexpr int row_threads() {
   return K::NC > 54 ? 256 : 512;
 }
+template <class K>
+constexpr int row_waves() {
+  return K::NC <= 3 ? 6 : K::NC <= 9 ? 4 : 1;
+}
 template <int LA, int LB, int LC, int LD, class R, bool XL>
-__global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_kernel(RowLaunch a) {
+__global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>()),
+                                        (row_waves<Cls<LA, LB, LC, LD>>())) void eri_row_kernel(RowLaunch a) {
   using K = Cls<LA, LB, LC, LD>;
-  constexpr int kRowThreads = row_threads<K>();
+  const int nthread = blockDim.x;  // see row_block
   constexpr int NROW = K::NCA + K::NCB, NAB = K::NCA * K::NCB, NCD = K::NCC * K::NCD;
   extern __shared__ double s_rows[];
-  __shared__ R s_tab[rys_tab_len(K::NR)];
+  using Rys = RysRow<K::NR, R, K::NC == 1, XL>;
+  __shared__ alignas(16) R s_tab[Rys::kLen];
   __shared__ unsigned s_queue[kRowChunk];  // surviving kets, most primitive pairs first
   __shared__ int s_hist[kRowBuckets];
   __shared__ double s_jab[kRowJ * NAB];
@@ -160,8 +172,8 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
   __shared__ double s_psum;
   const int tid = threadIdx.x, lane = tid & 63;
   {
-    const R *g = rys_table<R>(a.rys, a.rys32) + rys_tab_off(K::NR);
-    for (int e = tid; e < rys_tab_len(K::NR); e += kRowThreads) s_tab[e] = g[e];
+    const R *g = rys_table<R>(Rys::kHalf ? a.rys_half : a.rys, a.rys32_half);
+    for (int e = tid; e < Rys::kLen; e += nthread) s_tab[e] = g[Rys::src(e)];
     if (tid == 0) {
       s_tot[0] = s_tot[1] = 0;
       s_psum = 0.0;
@@ -202,16 +214,16 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
     const ScreenArgs sa{a.Bg, a.Bm, a.mol_boff, a.mol_ns, a.nmat, a.thresh, a.screen};
     int ncand = 0;
     double psum = 0.0;
-    constexpr int kPer = kRowChunk / kRowThreads;
+    constexpr int kPer = kRowChunk / 256;
     unsigned mine[kPer];  // ket, contractions
     int place[kPer];      // bucket and rank in it (< 0: none)
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int t = tid + u * kRowThreads, j = j0 + t;
+      const int t = tid + u * nthread, j = j0 + t;
       bool pass = false, cand = false;
       unsigned mask = 0;
       int kk = 0, npp = 0;
-      if (j < j1) {
+      if (t < kRowChunk && j < j1) {
         const PairScr Q = a.kscr[j];
         npp = a.ket[j].npp;
         const double qq = P.Q * Q.Q;
@@ -261,7 +273,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
     // chunk, whose digestion then uses every lane; up to 64 where a bra has a
     // handful of kets); kets [end[l + 1], end[l]) of the queue get 2^l lanes.
     work = __builtin_amdgcn_readfirstlane(work);
-    const int turns = max(1, work / kRowThreads);
+    const int turns = max(1, work / nthread);
     int end[8], nunit = 0;
     end[0] = n;
     end[7] = 0;
@@ -277,7 +289,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
     // each: a chain of 64 bra primitives is 8 long in a small molecule
     const int nb = bp->npp;
     int nsplit = 1;
-    while (2 * nsplit * nunit <= kRowThreads / 64 && nb >= 4 * nsplit) nsplit *= 2;
+    while (2 * nsplit * nunit <= nthread / 64 && nb >= 4 * nsplit) nsplit *= 2;
     // the molecule's planes; density rows in, exchange rows cleared
     const bool one = a.nmol == 1;
     const ConstPtr<MolPlanes> mp = as_const(a.mols + (one ? 0 : mol));
@@ -289,7 +301,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
       const GlobalDouble *x = (const GlobalDouble *)(one ? a.m0.kx[rp.kind] : mp->kx[rp.kind]) + rp.idx;
       const int S = a.kps[rp.kind];
       double *xs = s_x + p * NROW * w, *ks = s_k + p * NROW * w;
-      for (int c = tid; c < w; c += kRowThreads) {
+      for (int c = tid; c < w; c += nthread) {
         const int f = colmap[c];
         if (f < 0) continue;
 #pragma unroll
@@ -301,7 +313,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
         }
       }
     }
-    for (int e = tid; e < a.nj * NAB; e += kRowThreads) s_jab[e] = 0.0;
+    for (int e = tid; e < a.nj * NAB; e += nthread) s_jab[e] = 0.0;
     __syncthreads();
     const int pa = bp->a, pb = bp->b;
     const double bra_scale = 0.5 * (pa == pb ? 1.0 : 2.0);
@@ -346,7 +358,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
       R I[K::NC];
 #pragma unroll
       for (int o = 0; o < K::NC; ++o) I[o] = 0;
-      eval_bra<LA, LB, LC, LD, R>(a.prims, a.primc32, s_tab, bp, nb * part / nsplit, nb * (part + 1) / nsplit, Cc, CD,
+      eval_bra<LA, LB, LC, LD, R, XL>(a.prims, a.primc32, s_tab, bp, nb * part / nsplit, nb * (part + 1) / nsplit, Cc, CD,
                                   koff, nkp, g, G, I);
       for (int off = G >> 1; off > 0; off >>= 1) {
 #pragma unroll
@@ -414,7 +426,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
       const int S = a.kps[rp.kind];
       const double *ks = s_k + p * NROW * w;
       const double coef = 0.5 * rp.sign;
-      for (int c = tid; c < w; c += kRowThreads) {
+      for (int c = tid; c < w; c += nthread) {
         const int f = colmap[c];
         if (f < 0) continue;
 #pragma unroll
@@ -427,7 +439,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
         }
       }
     }
-    for (int e = tid; e < a.nj * NAB; e += kRowThreads) {
+    for (int e = tid; e < a.nj * NAB; e += nthread) {
       const double v = s_jab[e];
       if (v != 0.0) unsafeAtomicAdd(a.ja_bra + (size_t)e * a.nbra + i, a.jcoef[e / NAB] * v);
     }
@@ -440,16 +452,34 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>())) void eri_row_
   }
 }
 
-// LDS of a block in bytes: the static arrays (with padding) and sets sets of
-// rows (exchange, and density)
-template <class K, class R>
-size_t row_lds(int nk, int width, int sets) {
-  const size_t fixed = sizeof(R) * rys_tab_len(K::NR) + 4 * (kRowChunk + kRowBuckets) + 8 * kRowJ * K::NCA * K::NCB + 256;
-  return fixed + (size_t)sets * nk * (K::NCA + K::NCB) * width * sizeof(double);
+// LDS of a block in bytes: the static arrays (with padding), the exchange rows
+// and, with XL, the density rows
+template <class K, class R, bool XL>
+size_t row_lds(int nk, int width) {
+  const size_t fixed = sizeof(R) * RysRow<K::NR, R, K::NC == 1, XL>::kLen + 4 * (kRowChunk + kRowBuckets) + 8 * kRowJ * K::NCA * K::NCB + 256;
+  return fixed + (size_t)(XL ? 2 : 1) * nk * (K::NCA + K::NCB) * width * sizeof(double);
 }
 
 constexpr size_t kRowLdsMax = 160 * 1024;
 constexpr long long kRowGrid = 8192;
+
+// Threads of a block of the launch: the size that keeps more wavefronts on a
+// CU, as its registers (of the kernel) and LDS allow; the smaller of two that
+// keep as many, since its blocks screen while others evaluate.  C40H82 / 6-31G(d), ms a
+// launch, 256 and 512 threads: (ss|ss), equal wavefronts, 2.18 and 2.27;
+// (pp|ps), with rows that leave room for two blocks, 1.07 and 1.23; with rows
+// that leave room for one (dp|ps) 1.67 and 1.38, (dd|ss) 0.61 and 0.45; 32
+// water clusters, mixed, 26.7 -> 22.3 ms a build.  A launch of few items
+// leaves CUs idle whatever the size and takes the larger one ((H2O)4 /
+// cc-pVDZ, up to 406 items a launch, 0.69 -> 0.61 ms a build; with the line
+// at 1024 the launches of (H2O)6 / cc-pVTZ lose, 9.39 -> 9.60).
+constexpr long long kRowFew = 512;
+inline int row_block(int most, int vgprs, size_t lds, long long items) {
+  if (most <= 256 || items <= kRowFew) return most;
+  const int per_cu = 4 * std::min(8, 512 / ((std::max(vgprs, 1) + 7) / 8 * 8));  // wavefronts
+  auto waves = [&](int n) { return std::min<int>((int)(kRowLdsMax / lds), per_cu / (n / 64)) * (n / 64); };
+  return waves(512) > waves(256) ? 512 : 256;
+}
 
 template <int LA, int LB, int LC, int LD, class R, bool XL>
 hipError_t launch_row_x(const RowLaunch &a, hipStream_t s) {
@@ -457,14 +487,19 @@ hipError_t launch_row_x(const RowLaunch &a, hipStream_t s) {
   auto kern = eri_row_kernel<LA, LB, LC, LD, R, XL>;
   static std::once_flag once;  // allow dynamic LDS beyond the default limit, once per instantiation
   static hipError_t attr = hipSuccess;
+  static int vgprs = 0;
   std::call_once(once, [&] {
+    hipFuncAttributes fa{};
+    attr = hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(kern));
+    if (attr != hipSuccess) return;
+    vgprs = fa.numRegs;
     attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               160 * 1024 - (int)row_lds<K, R>(0, 0, 0));
+                               160 * 1024 - (int)row_lds<K, R, XL>(0, 0));
   });
   if (attr != hipSuccess) return attr;
   const long long items = (long long)a.nbra * a.nchunk;
   const size_t dyn = (size_t)(XL ? 2 : 1) * a.nk * (K::NCA + K::NCB) * a.width * sizeof(double);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(items < kRowGrid ? items : kRowGrid)), dim3(row_threads<K>()), dyn, s, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(items < kRowGrid ? items : kRowGrid)), dim3(row_block(row_threads<K>(), vgprs, row_lds<K, R, XL>(a.nk, a.width), items)), dyn, s, a);
   return hipGetLastError();
 }
 
@@ -474,8 +509,8 @@ hipError_t launch_row_cls(const RowLaunch &a, hipStream_t s) {
   if ((long long)a.nbra * a.nchunk <= 0) return hipSuccess;
   // density rows in LDS where both sets fit: GHF (H2O)16 (eight planes)
   // takes the second form for (ps|ps) and up, 11.5 -> 9.4 ms a build with it
-  if (row_lds<K, R>(a.nk, a.width, 2) <= kRowLdsMax) return launch_row_x<LA, LB, LC, LD, R, true>(a, s);
-  if (row_lds<K, R>(a.nk, a.width, 1) <= kRowLdsMax) return launch_row_x<LA, LB, LC, LD, R, false>(a, s);
+  if (row_lds<K, R, true>(a.nk, a.width) <= kRowLdsMax) return launch_row_x<LA, LB, LC, LD, R, true>(a, s);
+  if (row_lds<K, R, false>(a.nk, a.width) <= kRowLdsMax) return launch_row_x<LA, LB, LC, LD, R, false>(a, s);
   return hipErrorInvalidValue;
 }
 
@@ -517,8 +552,8 @@ bool row_group_lds(int la, int lb, int lc, int ld, int fp32, int nk, int width, 
     return launch_row_prec<A, B, C, D>(a, s);
 #define CQX_ROW_LDS(A, B, C, D)                                             \
   if (la == A && lb == B && lc == C && ld == D) {                           \
-    bytes = fp32 ? row_lds<Cls<A, B, C, D>, float>(nk, width, 1)               \
-                 : row_lds<Cls<A, B, C, D>, double>(nk, width, 1);             \
+    bytes = fp32 ? row_lds<Cls<A, B, C, D>, float, false>(nk, width)               \
+                 : row_lds<Cls<A, B, C, D>, double, false>(nk, width);             \
     return true;                                                            \
   }
 

@@ -80,6 +80,65 @@ __device__ __forceinline__ void rys_roots_sec(R T, const R *__restrict__ tabn, R
   }
 }
 
+// The row kernels' own form of the table: LDS copies, read by every lane for
+// itself, 14 coefficients a value, keep the LDS (128 bytes a cycle and CU) as
+// busy as the ALUs where there is little else to do per quadrature point.  On
+// half intervals of T 11 terms leave the FP64 series' error at their rounding
+// (one root, largest relative error over the table 2.1e-16, mean 5.3e-17, as
+// with 14 on unit intervals), and 6 terms the FP32 one's (1.2e-7 both ways).
+// Layout [half interval][power][value]: nodes and weights of one power lie
+// side by side; an (ss|ss) class keeps the weights alone (WONLY).  The FP64
+// section of two roots grows from 20.6 to 32.4 KB, so a block that has no
+// room to spare (ROOM false) keeps unit intervals: 32 water clusters 27.0 ->
+// 25.5 ms a build, but GHF (H2O)16 / cc-pVDZ 8.6 -> 9.1, its (ds|ps) rows then
+// not fitting any more.  FP64 sections of three roots and more stay as they
+// are (35 -> 55 KB).
+template <int N, class R, bool WONLY, bool ROOM>
+struct RysRow {
+  static constexpr bool kF32 = sizeof(R) == 4;
+  static constexpr bool kHalf = kF32 || N == 1 || (N == 2 && ROOM);
+  static constexpr int kCoef = kF32 ? 6 : 11;
+  static constexpr int kVal = 2 * N, kFirst = WONLY ? N : 0, kKeep = kVal - kFirst;
+  static constexpr int kLen = kHalf ? (34 + 6 * N) * 2 * kCoef * kKeep : rys_tab_len(N);
+  // entry e of the LDS copy in the table
+  static __device__ __forceinline__ int src(int e) {
+    if (!kHalf) return rys_tab_off(N) + e;
+    int o = 0;
+    for (int k = 1; k < N; ++k) o += (34 + 6 * k) * 2 * kCoef * 2 * k;
+    return o + e / kKeep * kVal + kFirst + e % kKeep;
+  }
+};
+template <int N, class R, bool WONLY, bool ROOM>
+__device__ __forceinline__ void rys_roots_row(R T, const R *__restrict__ tabn, R *__restrict__ x, R *__restrict__ w) {
+  using S = RysRow<N, R, WONLY, ROOM>;
+  if constexpr (!S::kHalf) {
+    rys_roots_sec<N, R>(T, tabn, x, w);
+  } else if (T >= (R)(34 + 6 * N)) {
+    const R rs = eval_rsqrt<R>(T), rt = rs * rs;
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      x[r] = (R)cqx_rys_asym_x[N][r] * rt;
+      w[r] = (R)cqx_rys_asym_w[N][r] * rs;
+    }
+  } else {
+    const int i = (int)(T + T);
+    const R t = T - ((R)0.5 * (R)i + (R)0.25);
+    const R *c = tabn + i * (S::kCoef * S::kKeep);
+    R v[S::kKeep];
+#pragma unroll
+    for (int r = 0; r < S::kKeep; ++r) v[r] = c[(S::kCoef - 1) * S::kKeep + r];
+#pragma unroll
+    for (int k = S::kCoef - 2; k >= 0; --k)
+#pragma unroll
+      for (int r = 0; r < S::kKeep; ++r) v[r] = fma(t, v[r], c[k * S::kKeep + r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      if (!WONLY) x[r] = v[r];
+      w[r] = v[N - S::kFirst + r];
+    }
+  }
+}
+
 // All n roots and weights, n known at compile time.
 template <int N, class R>
 __device__ __forceinline__ void rys_roots(R T, const R *__restrict__ tab, R *__restrict__ x,
