@@ -18,9 +18,9 @@
 // - the quartet is digested by the block from LDS with each term's density
 //   block staged there first.
 // Measured, (H2O)2 / cc-pVQZ RHF J/K: (gg|gg) 11.4 -> 0.17 ms, (gg|gf) 6.1 ->
-// 0.16, the build 43 -> 15.9 ms; against the wave kernels it wins from about
-// 1000 components ((fd|dp) 0.52 against 0.65 ms; (dd|dp), 648, 0.44 against
-// 0.31).
+// 0.16, the build 43 -> 15.9 ms.  The wave kernels, built up to 1080
+// components, win below ((H2O)6 / cc-pVTZ: (fd|dp) 0.27 against 0.52 ms,
+// (dd|dp) 0.39 against 0.44).
 //
 // A quartet too large for LDS is split over ranges of its first shell's
 // components, each a work item of its own (a is the slowest index of the

@@ -72,8 +72,25 @@ constexpr int wave_lds_bytes() {
 // single quartet gives an update term fewer items than lanes (e.g. 18 for
 // (dp|ps) with one plane), so most lanes of a digestion step would idle
 // while it waits on memory.
+// Wavefronts per SIMD asked of the compiler.  From 216 components on it
+// would fetch the table entries of every root and output before the first
+// product and take 200 to 512 registers for them (with spills), which leaves
+// one or two wavefronts a SIMD and every quartet's chain of loads exposed.
+// There the roots are a rolled loop, each fetching its own entries, and the
+// registers are held to what the outputs and the 2D tables need.  (H2O)6 /
+// cc-pVTZ, us a launch: (dd|dp) 746 -> 385, (fp|dp) 639 -> 284, (fd|dp) 576 ->
+// 272, (dp|dp) 524 -> 341, (dd|dd) 298 -> 170; one more wavefront 421, 371,
+// 350, 423, 217, one fewer 416, 349, 464, 403, 179.  Below 216 unrolled roots
+// and the compiler's choice are no worse ((dp|pp) 390, rolled 412).
+constexpr int kWaveRolled = 216;
+template <class K>
+constexpr int wave_waves() {
+  return K::NC < kWaveRolled ? 1 : K::NC == kWaveRolled ? 3 : K::NC <= 400 ? 4 : K::NC <= 700 ? 3 : 2;
+}
+
 template <int LA, int LB, int LC, int LD, class R, int QT>
-__global__ __launch_bounds__(64 * kWavesPerBlock) void eri_wave_kernel(EriLaunch a) {
+__global__ __launch_bounds__((64 * kWavesPerBlock),
+                                        (wave_waves<Cls<LA, LB, LC, LD>>())) void eri_wave_kernel(EriLaunch a) {
   using K = Cls<LA, LB, LC, LD>;
   constexpr int NOWN = (K::NC + 63) / 64;
   constexpr int HSZ = 3 * K::NR * K::NH;
@@ -210,19 +227,26 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void eri_wave_kernel(EriLaunch
     wave_sync();
     for (int g = 0; g < cnt; ++g) {
       const int t = quartet_of(k0 + g);  // uniform across the wave
+      R s[NOWN];  // (outputs beyond the last repeat the first and are dropped)
 #pragma unroll
-      for (int k = 0; k < NOWN; ++k) {
-        if (lane + 64 * k >= K::NC) continue;
-        R s = 0;
+      for (int k = 0; k < NOWN; ++k) s[k] = 0;
+      auto add_root = [&](const R *Hr) {
 #pragma unroll
-        for (int r = 0; r < K::NR; ++r) {
-          const R *Hr = H + g * HSZ + r * 3 * K::NH;
-          s = fma(Hr[ox[k]] * Hr[oy[k]], Hr[oz[k]], s);
-        }
+        for (int k = 0; k < NOWN; ++k) s[k] = fma(Hr[ox[k]] * Hr[oy[k]], Hr[oz[k]], s[k]);
+      };
+      const R *Hg = H + g * HSZ;
+      if constexpr (K::NC < kWaveRolled) {
+#pragma unroll
+        for (int r = 0; r < K::NR; ++r) add_root(Hg + r * 3 * K::NH);
+      } else {
+#pragma unroll 1
+        for (int r = 0; r < K::NR; ++r) add_root(Hg + r * 3 * K::NH);
+      }
+#pragma unroll
+      for (int k = 0; k < NOWN; ++k)
 #pragma unroll
         for (int u = 0; u < QT; ++u)
-          if (u == t) acc[u][k] += s;
-      }
+          if (u == t) acc[u][k] += s[k];
     }
     wave_sync();
   }
