@@ -46,6 +46,33 @@ namespace cqx {
 
 namespace {
 
+// Sums of N values over the wave, added to out: while a lane holds several
+// values it gives half of them to its partner and takes the partner's share of
+// the rest, so N values cost about N + 4 exchanges instead of 6 N.  (With six
+// each, the J(a, b) sums of C40H82 / 6-31G(d) took 0.28 of 1.29 ms of
+// (dp|ss) and 0.14 of 0.45 of (dd|ss).)
+template <int N, int O>
+__device__ __forceinline__ void wave_sums_add(const double (&v)[N], int base, int most, double *out, int lane) {
+  if constexpr (O == 0) {
+    if (base < most) unsafeAtomicAdd(out + base, v[0]);
+  } else if constexpr (N == 1) {
+    double s = v[0];
+#pragma unroll
+    for (int o = O; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (base < most && (lane & (2 * O - 1)) == 0) unsafeAtomicAdd(out + base, s);
+  } else {
+    constexpr int H = (N + 1) / 2;
+    const bool up = (lane & O) != 0;
+    double keep[H];
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const double hi = H + i < N ? v[H + i < N ? H + i : 0] : 0.0;  // (a slot beyond the last adds nothing)
+      keep[i] = (up ? hi : v[i]) + __shfl_xor(up ? v[i] : hi, O);
+    }
+    wave_sums_add<H, O / 2>(keep, base + (up ? H : 0), most, out, lane);
+  }
+}
+
 // Buckets of the surviving kets by their primitive pairs: exact up to 32,
 // then in fours, the last one open.  bucket_most: the most primitive pairs of
 // a bucket (of the open one a stand-in: it takes the most lanes anyway).
@@ -400,17 +427,23 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>()),
         double t[NCD];
 #pragma unroll
         for (int e = 0; e < NCD; ++e) t[e] = 0.0;
+        // J(a, b) sums formed together (a divisor of NAB)
+        constexpr int NS = NAB <= 10 ? NAB : NAB % 9 == 0 ? 9 : NAB % 10 == 0 ? 10 : 5;
 #pragma unroll
-        for (int ab = 0; ab < NAB; ++ab) {
-          const double xab = as_const(a.jx_bra)[(size_t)(p * NAB + ab) * a.nbra + i];
-          double s = 0.0;
+        for (int ab0 = 0; ab0 < NAB; ab0 += NS) {
+          double s[NS];
 #pragma unroll
-          for (int e = 0; e < NCD; ++e) {
-            s = fma(Id[ab * NCD + e], x[e], s);
-            t[e] = fma(Id[ab * NCD + e], xab, t[e]);
+          for (int k = 0; k < NS; ++k) {
+            const int ab = ab0 + k;
+            const double xab = as_const(a.jx_bra)[(size_t)(p * NAB + ab) * a.nbra + i];
+            s[k] = 0.0;
+#pragma unroll
+            for (int e = 0; e < NCD; ++e) {
+              s[k] = fma(Id[ab * NCD + e], x[e], s[k]);
+              t[e] = fma(Id[ab * NCD + e], xab, t[e]);
+            }
           }
-          s = wave_sum(s);
-          if (lane == 0) unsafeAtomicAdd(&s_jab[p * NAB + ab], s);
+          wave_sums_add<NS, 32>(s, 0, NS, s_jab + p * NAB + ab0, lane);
         }
         if (on)
 #pragma unroll
