@@ -28,7 +28,11 @@
 //
 // Measured against the quartet-list build (ms a build, two bins): C40H82
 // 90.5 -> 36.9, mixed 71.5 -> 30.8; the batch 75 -> 38; GHF (H2O)16 / cc-pVDZ
-// 12.8 -> 9.4; (H2O)7 3.2 -> 2.0; (H2O)4 1.38 -> 1.10.
+// 12.8 -> 9.4; (H2O)7 3.2 -> 2.0; (H2O)4 1.38 -> 1.10.  With the later changes
+// noted below and the front's C40H82 takes 23.9, mixed 20.5, the batch 20.4,
+// GHF 8.6, (H2O)7 1.15, (H2O)4 0.57.  What bounds them now: about half of the
+// VALU's cycles at three wavefronts a SIMD (chains of reciprocal square root,
+// table read and Horner steps), the LDS 25 to 50 % busy with the table.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -219,7 +223,7 @@ __global__ __launch_bounds__((row_threads<Cls<LA, LB, LC, LD>>()),
     const int j0 = lo + ch * kRowChunk, j1 = min(hi, j0 + kRowChunk);
     if (j0 >= j1) continue;
     // candidates: the Schwarz pre-cut prefix of the molecule's kets (Q
-    // descending), as in cand_count_kernel; the precision split is monotonic
+    // descending), as in candidates_kernel; the precision split is monotonic
     // in the ket index too
     const double Qi = bp->Q;
     double need = 0.0;
