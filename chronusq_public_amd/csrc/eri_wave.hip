@@ -50,19 +50,29 @@ bool eri_wave_qt_built(int la, int lb, int lc, int ld, int fp32, int qt) {
   }
 }
 
-// 4 quartets per wave for Cartesian quartets of at most 108 components, 2
-// up to 216, else 1 (measured on the GHF and C40H82 builds)
+// 4 quartets per wave for Cartesian quartets of at most 162 components, 2 up
+// to 400, else 1: a wave's quartets share the waits of one chain of loads.
+// A list too short for kFewWaves waves (four a SIMD) takes fewer.  Measured
+// with 108 and 216 as the lines whatever the list, and as here (ms a build):
+// (H2O)6 / cc-pVTZ 7.54 -> 7.27, 32 molecules mixed 20.5 -> 19.9, C40H82 /
+// 6-31G(d) 24.05 -> 23.8, (H2O)4 / cc-pVDZ 0.570 -> 0.562; without the rule
+// for short lists water / 6-31G(d) loses, 0.390 -> 0.406.  Two for every larger
+// class gives no more (C40H82 24.0, cc-pVTZ 7.28).
+constexpr long long kFewWaves = 4096;
 int eri_wave_default_qt(int la, int lb, int lc, int ld) {
   auto nc = [](int l) { return (l + 1) * (l + 2) / 2; };
   const int n = nc(la) * nc(lb) * nc(lc) * nc(ld);
-  return n <= 108 ? 4 : n <= 216 ? 2 : 1;
+  return n <= 162 ? 4 : n <= 400 ? 2 : 1;
 }
 
 hipError_t launch_eri_wave(const EriLaunch &a, hipStream_t s) {
   if (a.nq <= 0) return hipSuccess;
   if (a.store_mode) return hipErrorNotSupported;
   int qt = a.force_qt;
-  if (!eri_wave_qt_built(a.la, a.lb, a.lc, a.ld, a.fp32, qt)) qt = eri_wave_default_qt(a.la, a.lb, a.lc, a.ld);
+  if (!eri_wave_qt_built(a.la, a.lb, a.lc, a.ld, a.fp32, qt)) {
+    qt = eri_wave_default_qt(a.la, a.lb, a.lc, a.ld);
+    while (qt > 1 && a.nq < kFewWaves * qt) qt /= 2;
+  }
   if (max_l(a.la, a.lb, a.lc, a.ld) >= 3) {
     if (!eri_wave_qt_built(a.la, a.lb, a.lc, a.ld, a.fp32, qt)) qt = 1;
     if (max_l(a.la, a.lb, a.lc, a.ld) == 4)
