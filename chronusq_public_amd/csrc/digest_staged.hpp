@@ -55,17 +55,21 @@ struct DigestPlanes {  // one molecule's arrays of one kind
   int n, stride, p0, np, lgp;
 };
 
-// Stage block B of quartets [0, nq) (first functions sbf, E elements each):
-// the value of (quartet q, element e, plane p) goes to
-// sX[((q E + off(B) + e) << lgp) + p].
+// Stage block B of the quartets of molecule mol (whose planes P are) among
+// [0, nq) (first functions sbf, E elements each): the value of (quartet q,
+// element e, plane p) goes to sX[((q E + off(B) + e) << lgp) + p].  Another
+// molecule's functions may lie beyond the end of these planes: its quartets
+// are left for their own turn.
 template <class K, int B, int E>
-__device__ __forceinline__ void stage_block(const int (*__restrict__ sbf)[4], int nq, bool both,
-                                            const DigestPlanes &P, double *__restrict__ sX, int lane) {
+__device__ __forceinline__ void stage_block(const int (*__restrict__ sbf)[4], const int *__restrict__ smol, int mol,
+                                            int nq, bool both, const DigestPlanes &P, double *__restrict__ sX,
+                                            int lane) {
   using L = XLayout<K>;
   constexpr int R = kXRoles[B][0], C = kXRoles[B][1], NR = K::n(R), SZ = L::size(B);
   const int items = (nq * SZ) << P.lgp;
   for (int it = lane; it < items; it += 64) {
     const int p = it & ((1 << P.lgp) - 1), r = it >> P.lgp, q = r / SZ, e = r - q * SZ;
+    if (smol[q] != mol) continue;
     const int row = sbf[q][R] + e % NR, col = sbf[q][C] + e / NR;
     double v = 0.0;
     if (p < P.np) {
@@ -164,7 +168,7 @@ __device__ __forceinline__ void digest_staged(const double *sI, const int (*sbf)
         const DigestPlanes P = planes_of(kind);
         double *X = sX + xoff;
         xoff += (n * L::per_kind(kind)) << P.lgp;
-#define CQX_STAGE(B, E) stage_block<K, B, E>(tbf, n, kind == kJNonHer, P, X, lane)
+#define CQX_STAGE(B, E) stage_block<K, B, E>(tbf, tmol, mol, n, kind == kJNonHer, P, X, lane)
         if (kind == kJHer || kind == kJNonHer) {
           CQX_STAGE(0, L::EJ);
           CQX_STAGE(1, L::EJ);
