@@ -349,6 +349,15 @@ void join_sides(cqx_ctx *c, int nst) {
   }
 }
 
+// After a failure part way through a build: launches on the side streams may
+// still add into the context's buffers, which the next build clears on the
+// context stream alone, so they end before the call returns.
+void settle(cqx_ctx *c) {
+  for (hipStream_t t : c->side)
+    if (t) (void)hipStreamSynchronize(t);
+  (void)hipStreamSynchronize(c->stream);
+}
+
 // contraction signature: what the recorded launches depend on besides the
 // densities themselves
 std::string contraction_key(int screen, int is_complex, int ncon, const cqx_contraction *list) {
@@ -2625,8 +2634,10 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
     c->ws_scratch_peak = scratch_peak;
     c->stats.workspace_bytes = scr ? (long long)scratch_peak : (long long)workspace_bytes(c);
   } catch (const Unsupported &e) {
+    settle(c);
     return fail(c, CQX_ERR_UNSUPPORTED, e.what());
   } catch (const std::exception &e) {
+    settle(c);
     return fail(c, CQX_ERR_HIP, e.what());
   }
   c->stats.ms_total =
@@ -2876,6 +2887,7 @@ int cqx_grad_two_body_contract(cqx_ctx *c, int ngrad, int nmat, const cqx_contra
     HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->stats.ms_eri = ms;
   } catch (const std::exception &e) {
+    settle(c);
     return fail(c, CQX_ERR_HIP, e.what());
   }
   c->stats.ms_total =
