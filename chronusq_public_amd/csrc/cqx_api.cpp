@@ -135,8 +135,10 @@ template <class T>
 struct DevBuf {
   T *p = nullptr;
   size_t n = 0;
+  unsigned gen = 0;  // changes with the memory behind p
   void ensure(size_t m) {
     if (m <= n) return;
+    ++gen;
     if (p) (void)hipFree(p);
     p = nullptr;
     n = 0;
@@ -214,9 +216,12 @@ struct cqx_ctx {
   DevBuf<const double *> d_px;
   DevBuf<double *> d_pa;
   DevBuf<double> d_small;
-  // what the tables above (and the plane table) last held, so that a build
-  // with the same ones uploads nothing
-  std::vector<char> kept_cands, kept_px, kept_pa, kept_molplanes, kept_lists, kept_lstart;
+  // what the tables above (and the plane table) last received, and in which
+  // memory, so that a build with the same ones uploads nothing
+  struct Kept {
+    std::vector<char> bytes;
+    unsigned gen = 0;
+  } kept_cands, kept_px, kept_pa, kept_molplanes, kept_lists, kept_lstart;
   std::vector<cqx::MolInfo> molinfo;  // nmol + 1: the last entry holds the totals
   DevBuf<cqx::MolInfo> d_molinfo;
   DevBuf<cqx::ListLaunch> d_lists;
@@ -1453,17 +1458,18 @@ T *ws_upload(DevBuf<T> &buf, Arena *scr, const std::vector<T> &v, hipStream_t s,
 // The same for a table that rarely changes between builds of a context: kept
 // holds the bytes the context's buffer last received.
 template <class T>
-T *ws_upload_kept(DevBuf<T> &buf, std::vector<char> &kept, Arena *scr, const std::vector<T> &v, hipStream_t s,
+T *ws_upload_kept(DevBuf<T> &buf, cqx_ctx::Kept &kept, Arena *scr, const std::vector<T> &v, hipStream_t s,
                   const char *what) {
   if (scr) return ws_upload(buf, scr, v, s, what);
   const size_t n = sizeof(T) * v.size();
-  if (buf.p && buf.n >= v.size() && kept.size() == n && (n == 0 || std::memcmp(kept.data(), v.data(), n) == 0))
-    return buf.p;
-  kept.clear();
   buf.ensure(std::max<size_t>(v.size(), 1));
+  if (kept.gen == buf.gen && kept.bytes.size() == n && (n == 0 || std::memcmp(kept.bytes.data(), v.data(), n) == 0))
+    return buf.p;
+  kept.bytes.clear();
+  kept.gen = buf.gen;
   std::vector<char> bytes(reinterpret_cast<const char *>(v.data()), reinterpret_cast<const char *>(v.data()) + n);
   if (n) HIPCHK(hipMemcpyAsync(buf.p, bytes.data(), n, hipMemcpyHostToDevice, s));
-  kept.swap(bytes);  // the copy's source stays in place
+  kept.bytes.swap(bytes);  // the copy's source stays in place
   return buf.p;
 }
 template <class T>
@@ -2328,8 +2334,8 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
             if (lls[k].out32) counts[np + k] = (unsigned long long)batch[k].ncand;
           }
         } else {
-          c->kept_lists.clear();
-          c->kept_lstart.clear();
+          c->kept_lists.bytes.clear();
+          c->kept_lstart.bytes.clear();
           HIPCHK(hipMemcpyAsync(w.lists, lls.data(), sizeof(cqx::ListLaunch) * np, hipMemcpyHostToDevice, s));
           HIPCHK(hipMemcpyAsync(w.lstart, lstart.data(), sizeof(long long) * (np + 1), hipMemcpyHostToDevice, s));
           HIPCHK(cqx::launch_quartet_lists(w.lists, w.lstart, (int)np, lstart[np], s));

@@ -1,6 +1,7 @@
 """CPU tests of the host side of a build on a HIP runtime without a device
 (tests/cpp/fake_hip.cpp: kernels do nothing, streams and events are followed):
-a build that fails part way through leaves nothing in flight."""
+a build that fails part way through leaves nothing in flight, and the next one
+on the same context starts from tables it has uploaded itself."""
 import ctypes as C
 import os
 import subprocess
@@ -9,7 +10,7 @@ import sys
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-CASES = ["nothing_in_flight"]
+CASES = ["nothing_in_flight", "tables_after_failure"]
 
 
 def _cont(cqx, np, nb, n):
@@ -66,6 +67,28 @@ def _child(fakelib, case):
             read_back(word)
             failing(run)
             read_back(0)
+    elif case == "tables_after_failure":
+        def run(k):
+            tpi = tpi_of()
+            tpi.set_option("rows", 0)  # lists for every class pair, none with a candidate
+            assert _contract(cqx, np, tpi) is None
+            tpi.set_option("rows", 1)  # a small build: its tables are kept
+            assert _contract(cqx, np, tpi) is None
+            tpi.set_option("rows", 0)  # every list with candidates: larger tables
+            fake.fake_fail_malloc(C.c_longlong(k))
+            read_back(5)
+            e = _contract(cqx, np, tpi)
+            read_back(0)
+            fake.fake_fail_malloc(C.c_longlong(0))
+            tpi.set_option("rows", 1)
+            assert _contract(cqx, np, tpi) is None
+            assert fake.fake_unwritten_tables() == 0, (k, e)
+            return e
+
+        k = 0
+        while run(k := k + 1) is not None:
+            pass
+        assert k > 1
     print("child ok")
 
 
