@@ -1543,6 +1543,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       const cqx_contraction *L = list + start;  // molecule 0's contractions of the group
       const GroupPlan gp = plan_group(c, L, nmat, is_complex);
       if (scr) scr->used = 0;  // each group reuses the whole region
+      float group_ms = 0.0f;  // ERI launches of this group
       // densities (and, when allocating, the outputs) on the device:
       // molecule m's nmat matrices at xoff[m]
       std::vector<size_t> xoff(nmol + 1, 0);
@@ -2420,7 +2421,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         HIPCHK(hipEventSynchronize(c->ev1));
         float ms = 0.0f;
         HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        eri_ms_total += ms;
+        group_ms += ms;
       }
       if (!tiles_done) {  // no quartet-list batch: the tile lists' launches alone
         HIPCHK(hipEventRecord(c->ev0, s));
@@ -2433,7 +2434,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         HIPCHK(hipEventSynchronize(c->ev1));
         float ms = 0.0f;
         HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        eri_ms_total += ms;
+        group_ms += ms;
       }
       ensure_side(nst_all);
       if (nrow) {
@@ -2482,7 +2483,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       if (nrow) {
         float ms = 0.0f;  // with the list launches beside the row launches
         HIPCHK(hipEventElapsedTime(&ms, c->ev_r0, c->ev1));
-        eri_ms_total = ms;
+        group_ms = ms;
         row_slots.clear();
         for (int f = 0; f < qmul; ++f)
           for (const auto &rc : rcps) {
@@ -2494,6 +2495,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
           }
         add_row_stats(c, row_slots, rcount, pure_d, is_complex ? 2 : 1, nJ, nK);
       }
+      eri_ms_total += group_ms;
       if (scr) scratch_peak = std::max(scratch_peak, scr->used);
       // Record the same build into a graph for the next calls (option
       // graph; one contraction group and one list batch).  Capacities are

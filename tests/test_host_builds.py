@@ -1,7 +1,8 @@
 """CPU tests of the host side of a build on a HIP runtime without a device
 (tests/cpp/fake_hip.cpp: kernels do nothing, streams and events are followed):
 a build that fails part way through leaves nothing in flight, and the next one
-on the same context starts from tables it has uploaded itself."""
+on the same context starts from tables it has uploaded itself; the times of a
+call's contraction groups add up."""
 import ctypes as C
 import os
 import subprocess
@@ -10,7 +11,7 @@ import sys
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-CASES = ["nothing_in_flight", "tables_after_failure"]
+CASES = ["nothing_in_flight", "tables_after_failure", "groups_add_up"]
 
 
 def _cont(cqx, np, nb, n):
@@ -89,6 +90,11 @@ def _child(fakelib, case):
         while run(k := k + 1) is not None:
             pass
         assert k > 1
+    else:
+        tpi = tpi_of()
+        for n, groups in ((2, 1), (8, 1), (9, 2), (20, 3)):
+            assert _contract(cqx, np, tpi, n) is None
+            assert tpi.last_stats()["ms_eri"] == groups  # every interval lasts 1 ms
     print("child ok")
 
 
