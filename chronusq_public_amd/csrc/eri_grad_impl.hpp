@@ -264,8 +264,9 @@ __global__ __launch_bounds__((GradWave<LA, LB, LC, LD>::NT)) void grad_wave_kern
       j = (int)(q - (long long)i * a.nket);
     }
     const PairRec bp = a.bra[i], kp = a.ket[j];
-    for (int e = tid; e < 9 * K::NC; e += W::NT) s_d[e] = 0.0;
     const int nk = kp.npp, ntot = bp.npp * nk;
+    if (ntot == 0) continue;  // (the barriers between clearing and reading the sums are those of the loop below)
+    for (int e = tid; e < 9 * K::NC; e += W::NT) s_d[e] = 0.0;
     const int grp = tid / (3 * W::NR), sub = tid - grp * (3 * W::NR), root = sub / 3, d = sub - root * 3;
     for (int k0 = 0; k0 < ntot; k0 += W::PP) {
       const int cnt = min(W::PP, ntot - k0);

@@ -76,7 +76,7 @@ int run_case(const char *name, const int (&nbc)[2], const int (&mols)[kQuartets]
     }
     mask[q] = q == 0 ? 0xFFu : 0xFEu;  // contraction 0 screened out of the others
   }
-  host_wave::run([&](int lane) { digest_staged<K, kXCap>(I.data(), bf, mask, mols, nq, ps, X.data(), lane); });
+  host_wave::run(64, [&](int lane) { digest_staged<K, kXCap>(I.data(), bf, mask, mols, nq, ps, X.data(), lane); });
   // the same updates term by term
   const int st[4] = {K::NCB * K::NCC * K::NCD, K::NCC * K::NCD, K::NCD, 1};
   for (int q = 0; q < nq; ++q)

@@ -9,7 +9,7 @@ from conftest import ROOT
 
 def test_staged_digestion_stays_in_its_molecules_planes(tmp_path):
     exe, cpp = str(tmp_path / "staged_test"), os.path.join(ROOT, "tests", "cpp")
-    r = subprocess.run(["g++", "-std=c++20", "-O1", "-pthread", "-Wno-attributes", "-Wno-unknown-pragmas",
+    r = subprocess.run(["g++", "-std=c++17", "-O1", "-Wno-attributes", "-Wno-unknown-pragmas",
                         "-I", os.path.join(cpp, "wave"), "-I", os.path.join(ROOT, "chronusq_public_amd", "csrc"),
                         os.path.join(cpp, "staged_test.cpp"), "-o", exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
