@@ -80,27 +80,32 @@ def _write_values(name, tab):
     with open(path, "w") as f:
         for i in range(0, tab.size, 4):
             f.write(", ".join(float(v).hex() for v in tab[i:i + 4]) + ",\n")
-    return path
+
+
+def rys_tables():
+    """The tables the kernels read, by the name of the file that embeds each."""
+    raw = np.fromfile(os.path.join(CSRC, "rys_table.bin"), dtype="<f8")
+    return {"rys_table_data.inc": rys_powers(raw).astype(np.float64),
+            "rys_half_data.inc": rys_halves(raw, 2, 11).astype(np.float64),
+            "rys_half32_data.inc": rys_halves(raw, 3, 6).astype(np.float32)}
 
 
 def write_rys_inc():
-    raw = np.fromfile(os.path.join(CSRC, "rys_table.bin"), dtype="<f8")
-    _write_values("rys_half_data.inc", rys_halves(raw, 2, 11).astype(np.float64))
-    _write_values("rys_half32_data.inc", rys_halves(raw, 3, 6).astype(np.float32))
-    return _write_values("rys_table_data.inc", rys_powers(raw).astype(np.float64))
+    for name, tab in rys_tables().items():
+        _write_values(name, tab)
 
 
-# the sources of the ERI + digestion launches of a Fock build: the kernels,
-# their headers and the Rys table
-KERNEL_SOURCES = ("eri_", "digest", "kernels.", "device_types.hpp", "rys.hpp", "rys_table.bin", "front.",
-                  "limits.hpp")
+# the sources of the ERI + digestion launches of a Fock build: the kernels and
+# their headers (the Rys tables are hashed as derived)
+KERNEL_SOURCES = ("eri_", "digest", "kernels.", "device_types.hpp", "rys.hpp", "rys_table.h", "front.", "screen.",
+                  "tile_layout.hpp", "limits.hpp")
 
 
 def source_digest():
     """First 16 hex digits of a SHA-256 over the sources of the ERI and
-    digestion kernels (file names included).  Kernel profiles record it,
-    so that a profiled figure is reported only beside the kernels it was
-    measured on."""
+    digestion kernels (file names included) and the Rys tables.  Kernel
+    profiles record it, so that a profiled figure is reported only beside the
+    kernels it was measured on."""
     import hashlib
     h = hashlib.sha256()
     for f in sorted(os.listdir(CSRC)):
@@ -109,6 +114,9 @@ def source_digest():
         h.update(f.encode())
         with open(os.path.join(CSRC, f), "rb") as fh:
             h.update(fh.read())
+    for name, tab in sorted(rys_tables().items()):
+        h.update(name.encode())
+        h.update(tab.tobytes())
     return h.hexdigest()[:16]
 
 
