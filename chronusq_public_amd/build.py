@@ -98,7 +98,7 @@ def write_rys_inc():
 # the sources of the ERI + digestion launches of a Fock build: the kernels and
 # their headers (the Rys tables are hashed as derived)
 KERNEL_SOURCES = ("eri_", "digest", "kernels.", "device_types.hpp", "rys.hpp", "rys_table.h", "front.", "screen.",
-                  "tile_layout.hpp", "limits.hpp")
+                  "tile_layout.hpp", "cart_coef.hpp", "limits.hpp")
 
 
 def source_digest():

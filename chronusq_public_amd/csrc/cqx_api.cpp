@@ -100,11 +100,6 @@ constexpr size_t kGatherBytes = 1 << 20;
 // 10.27 -> 10.42 ms with 16 M)
 constexpr long long kSmallLists = 1 << 20;
 
-// LDS of a row block beyond which a class pair takes quartet lists: all a
-// block can have (one block per CU still beats the lists: GHF (ps|ps) of
-// (H2O)16 1.41 against 2.04 ms)
-constexpr size_t kRowLdsUse = 160 * 1024;
-
 constexpr int kNumClass = (cqx::kMaxLDev + 1) * (cqx::kMaxLDev + 2) / 2;  // (la, lb), la >= lb
 inline int class_of(int la, int lb) { return la * (la + 1) / 2 + lb; }
 inline void class_ls(int c, int &la, int &lb) {
@@ -1718,8 +1713,7 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         class_ls(ck, lc_, ld_);
         const int ncq = cqx::ncart(la_) * cqx::ncart(lb_) * cqx::ncart(lc_) * cqx::ncart(ld_);
         if (!(ncq <= c->fast_max_nc || (c->use_wave && c->fast_max_nc > 0))) return false;
-        const size_t b = cqx::eri_row_lds(la_, lb_, lc_, ld_, 0, row0.nk, c->row_width[ck]);
-        return b > 0 && b <= (size_t)kRowLdsUse;
+        return cqx::eri_row_lds(la_, lb_, lc_, ld_, 0, row0.nk, c->row_width[ck]) > 0;
       };
       if (rows_ok)
         for (int cb = 0; cb < kNumClass; ++cb)

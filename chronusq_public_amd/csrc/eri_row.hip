@@ -1,5 +1,4 @@
-// Dispatch of the row kernels (eri_row_impl.hpp) and the transforms of the
-// Coulomb planes between matrix and pair order.
+// Dispatch of the row kernels (eri_row_impl.hpp).
 #include <hip/hip_runtime.h>
 
 #include "eri_row.hpp"
@@ -22,15 +21,10 @@ bool row_lds_of(int la, int lb, int lc, int ld, int fp32, int nk, int width, siz
 
 }  // namespace
 
-bool eri_row_built(int la, int lb, int lc, int ld) {
-  size_t b = 0;
-  return row_lds_of(la, lb, lc, ld, 0, 0, 0, b);
-}
-
 size_t eri_row_lds(int la, int lb, int lc, int ld, int fp32, int nk, int width) {
   size_t b = 0;
   if (!row_lds_of(la, lb, lc, ld, fp32, nk, width, b)) return 0;
-  return b <= 160 * 1024 ? b : 0;
+  return b <= kRowLdsMax ? b : 0;
 }
 
 hipError_t launch_eri_row(const RowLaunch &a, hipStream_t s) {

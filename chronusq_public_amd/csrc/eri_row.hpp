@@ -61,9 +61,11 @@ struct RowLaunch {
   unsigned long long *count;    // quartets, candidates
   double *prim_sum;
 };
-// whether the class has a row kernel, and the LDS one block takes (0: more
-// than the device has)
-bool eri_row_built(int la, int lb, int lc, int ld);
+// LDS of a row block at most: all a block can have.  One block per CU still
+// beats quartet lists: GHF (ps|ps) of (H2O)16 1.41 against 2.04 ms.
+constexpr size_t kRowLdsMax = 160 * 1024;
+// the LDS one block takes (0: no row kernel for the class, or more than
+// kRowLdsMax)
 size_t eri_row_lds(int la, int lb, int lc, int ld, int fp32, int nk, int width);
 hipError_t launch_eri_row(const RowLaunch &a, hipStream_t s);
 

@@ -497,7 +497,6 @@ size_t row_lds(int nk, int width) {
   return fixed + (size_t)(XL ? 2 : 1) * nk * (K::NCA + K::NCB) * width * sizeof(double);
 }
 
-constexpr size_t kRowLdsMax = 160 * 1024;
 constexpr long long kRowGrid = 8192;
 
 // Threads of a block of the launch: the size that keeps more wavefronts on a
@@ -531,7 +530,7 @@ hipError_t launch_row_x(const RowLaunch &a, hipStream_t s) {
     if (attr != hipSuccess) return;
     vgprs = fa.numRegs;
     attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               160 * 1024 - (int)row_lds<K, R, XL>(0, 0));
+                               (int)(kRowLdsMax - row_lds<K, R, XL>(0, 0)));
   });
   if (attr != hipSuccess) return attr;
   const long long items = (long long)a.nbra * a.nchunk;

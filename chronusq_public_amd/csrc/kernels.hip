@@ -13,14 +13,13 @@
 
 #include <algorithm>
 
+#include "cart_coef.hpp"
 #include "kernels.hpp"
 #include "screen.hpp"
 
 namespace cqx {
 
 namespace {
-
-__device__ __forceinline__ int ncart_d(int l) { return (l + 1) * (l + 2) / 2; }
 
 __device__ __forceinline__ void atomic_add(double *p, double v) { unsafeAtomicAdd(p, v); }
 
@@ -256,23 +255,6 @@ __global__ __launch_bounds__(64 * kTileListWaves) void tile_lists_kernel(const T
   }
 }
 
-__device__ __forceinline__ int sph_off(int l) {
-  // sum_{k<l} (2k+1) ncart(k): 0, 1, 10, 40, 110
-  const int off[5] = {0, 1, 10, 40, 110};
-  return off[l];
-}
-
-// coefficient T(cart comp c, pure function m) of a shell
-__device__ __forceinline__ double tcoef(const CartMap &M, int s, int c, int m) {
-  if (!M.sh_pure[s]) return c == m ? 1.0 : 0.0;
-  const int l = M.sh_l[s];
-  return M.sph[sph_off(l) + m * ncart_d(l) + c];
-}
-
-__device__ __forceinline__ int nfunc(const CartMap &M, int s) {
-  return M.sh_pure[s] ? 2 * M.sh_l[s] + 1 : ncart_d(M.sh_l[s]);
-}
-
 __global__ void to_cart_kernel(CartMap M, const double *X, int cplx, double *Pre, double *Pim,
                                int ps) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -309,7 +291,7 @@ __global__ void from_cart_kernel(CartMap M, const double *A, int her, double *AX
   const int mu = (int)(t % M.nb), nu = (int)(t / M.nb);
   const int sm = M.bf_shell[mu], cm = M.bf_comp[mu];
   const int sn = M.bf_shell[nu], cn = M.bf_comp[nu];
-  const int ncm = ncart_d(M.sh_l[sm]), ncn = ncart_d(M.sh_l[sn]);
+  const int ncm = ncart_f(M.sh_l[sm]), ncn = ncart_f(M.sh_l[sn]);
   double a = 0.0, b = 0.0;
   for (int i = 0; i < ncm; ++i) {
     const double ti = tcoef(M, sm, i, cm);
