@@ -467,6 +467,27 @@ def host_leg(bench, steps, out, line):
     }
 
 
+LEGS = {"mixed": lambda n: mixed_comparison(n, 1), "batched": lambda n: batched_comparison(n, 2),
+        "serving": lambda n: serving(n)}
+
+
+def leg_command(name, size):
+    return [sys.executable, os.path.abspath(__file__), "--leg", name, str(size), "--streams", str(LAUNCH_STREAMS)]
+
+
+def child_leg(cmd, timeout=600):
+    """One leg in a process of its own, so that a fault in it does not take
+    the figures of the others along: its result, or {"error": ...}."""
+    import subprocess
+    try:
+        r = subprocess.run(cmd, stdout=subprocess.PIPE, text=True, timeout=timeout)
+    except subprocess.TimeoutExpired:
+        return {"error": f"no result within {timeout} s"}
+    if r.returncode:
+        return {"error": f"the leg's process ended with status {r.returncode}"}
+    return json.loads(r.stdout.strip().splitlines()[-1])
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -490,6 +511,8 @@ def main():
     ap.add_argument("--copy-mb", type=int, default=0,
                     help="also run one device-to-device copy of this many MiB (HBM "
                          "counter calibration for rocprofv3 --pmc runs)")
+    ap.add_argument("--leg", nargs=2, metavar=("NAME", "SIZE"),
+                    help="run one of the legs mixed, batched, serving alone and print its object")
     args = ap.parse_args()
     if args.gpus != 1:
         raise SystemExit("bench.py measures one GPU: the direct J/K engine runs one process "
@@ -498,6 +521,9 @@ def main():
     from chronusq_public_amd import cqx
     global LAUNCH_STREAMS
     LAUNCH_STREAMS = args.streams
+    if args.leg:
+        print(json.dumps(LEGS[args.leg[0]](int(args.leg[1]))), flush=True)
+        return
     bench = Build(args.workload, nocc=161 if args.workload == "alkane40" else 20)
     for o in args.opt:
         name, value = o.split("=", 1)
@@ -597,18 +623,21 @@ def main():
             "max_abs_d_vs_eager": float(max(np.abs(a - b).max() for a, b in zip(gout, out))),
         }
         tpi.set_option("graph", 0)
-    if args.mixed_steps > 0:
-        line["mixed"] = mixed_comparison(args.mixed_steps, 1)
-    if args.batch_mols > 0:
-        line["batched"] = batched_comparison(args.batch_mols, 2)
-    if args.serve_jobs > 0:
-        line["serving"] = serving(args.serve_jobs)
     if not args.no_cpu:
         progress("cpu baseline: oracle builds on the host cores")
         cb, err = cpu_baseline(gbs, mol, mats, types, cplx, out)
         line["cpu_baseline"] = cb
         line["max_abs_dJK_vs_oracle"] = err
+    failed = False
+    for name, size in (("mixed", args.mixed_steps), ("batched", args.batch_mols), ("serving", args.serve_jobs)):
+        if size > 0 and not failed:  # nothing more on the GPU after a leg that died
+            line[name] = child_leg(leg_command(name, size))
+            failed = "error" in line[name]
+            if failed:
+                progress(f"{name}: {line[name]['error']}")
     print(json.dumps(line), flush=True)
+    if failed:
+        sys.exit(1)
 
 
 if __name__ == "__main__":
