@@ -1474,6 +1474,15 @@ T *ws_take(DevBuf<T> &buf, Arena *scr, size_t n, const char *what) {
   return buf.p;
 }
 
+// Kernel family that lists of a class take without a tuned choice: 0
+// lane-group, 1 wave-per-quartet, 2 generic.
+int list_route(const cqx_ctx *c, int la, int lb, int lc, int ld) {
+  const int ncq = cqx::ncart(la) * cqx::ncart(lb) * cqx::ncart(lc) * cqx::ncart(ld);
+  if (ncq <= c->fast_max_nc && cqx::eri_lane_group_built(la, lb, lc, ld)) return 0;
+  if (c->use_wave && cqx::eri_wave_available(la, lb, lc, ld)) return 1;
+  return 2;
+}
+
 // The direct J/K build of a contraction list (directScaffoldNew,
 // direct.hpp:1412-2123).  scr == nullptr: the workspace lives in the
 // context's own buffers, grown on demand (and a build may be recorded into
@@ -1711,8 +1720,9 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
         int la_, lb_, lc_, ld_;
         class_ls(cb, la_, lb_);
         class_ls(ck, lc_, ld_);
-        const int ncq = cqx::ncart(la_) * cqx::ncart(lb_) * cqx::ncart(lc_) * cqx::ncart(ld_);
-        if (!(ncq <= c->fast_max_nc || (c->use_wave && c->fast_max_nc > 0))) return false;
+        // classes that the options send to the generic kernel stay there (and
+        // so in FP64, which is all it has)
+        if (c->fast_max_nc <= 0 || list_route(c, la_, lb_, lc_, ld_) == 2) return false;
         return cqx::eri_row_lds(la_, lb_, lc_, ld_, 0, row0.nk, c->row_width[ck]) > 0;
       };
       if (rows_ok)
@@ -2034,14 +2044,11 @@ int contract(cqx_ctx *c, int screen, int ncon, const cqx_contraction *list, int 
       // kernel family of a class: 0 lane-group, 1 wave-per-quartet, 2 generic;
       // f32 < 0 asks for the family without a tuned choice
       auto route = [&](int la, int lb, int lc, int ld, int f32 = -1) {
-        const int ncq = cqx::ncart(la) * cqx::ncart(lb) * cqx::ncart(lc) * cqx::ncart(ld);
         if (f32 >= 0 && dual(la, lb, lc, ld)) {
           auto it = c->tuned_lanes.find(class_key(la, lb, lc, ld, f32));
           if (it != c->tuned_lanes.end()) return it->second >= kWaveTag ? 1 : 0;
         }
-        if (ncq <= c->fast_max_nc && cqx::eri_lane_group_built(la, lb, lc, ld)) return 0;
-        if (c->use_wave && cqx::eri_wave_available(la, lb, lc, ld)) return 1;
-        return 2;
+        return list_route(c, la, lb, lc, ld);
       };
       // classes with an FP32 kernel: the lane-group and wave kernels of the
       // s/p/d classes (quartets with an f or g shell stay in FP64)

@@ -262,7 +262,8 @@ int cqx_grad_two_body_contract(cqx_ctx *ctx, int ngrad, int nmat, const cqx_cont
  * a class pair with a row kernel, whose rows of the build's exchange planes
  * fit in LDS, screens, evaluates and digests its quartets in one launch
  * without quartet lists; 0: quartet lists for every class pair;
- * allocation-free builds, and builds with "fast_lanes" set, always take
+ * allocation-free builds, builds with "fast_lanes" set, and class pairs that
+ * "fast_max_nc" or "use_wave" send to the generic kernel always take
  * lists).  Setting any option
  * drops a recorded graph. */
 int cqx_set_option(cqx_ctx *ctx, const char *name, double value);
